@@ -21,11 +21,13 @@
 //
 //    Instruction K order.  The f8f6f4 MFMA's lane group g holds K-chunks g
 //    and g + 4 of its row (K 16g .. 16g + 15 and 64 + 16g .. 64 + 16g + 15).
-//    Kernels that need that order (block scales; fp4's two MFMA per step;
-//    operands paired with register-loaded ones) store chunk c at slot
+//    Kernels that need that order (block scales; operands paired with
+//    register-loaded ones) store chunk c at slot
 //    kpair_slot(c) ^ slot_xor(r): chunks g and g + 4 then sit at slots 2g and
 //    2g + 1 (before the XOR), the measured conflict-free reads.  Their DMA
-//    lane l fetches chunk kpair_chunk((l % 8) ^ slot_xor(row)).
+//    lane l fetches chunk kpair_chunk((l % 8) ^ slot_xor(row)).  (The 128 x
+//    128 tiles with block scales keep the plain order under strip_xor and
+//    read chunks g and g + 4 instead: conflict-free too.)
 //
 // 2. Output tile order ("XCD-contiguous, grouped columns").
 //    The dispatcher hands workgroup b to XCD b % 8.  tile_of_block() first
