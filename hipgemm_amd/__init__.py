@@ -28,6 +28,7 @@ from typing import Optional
 __all__ = [
     "HipGemmError", "lib", "lib_path", "fp8_gemm_bf16", "fp8_gemm",
     "fp8_gemm_4wave_256x256x128", "gemm_raw", "select_variant", "split_columns",
+    "auto_tile",
     "variant_name", "version", "tile_order", "lds_slot", "lds_slot_kpair",
     "lds_stage_slot",
     "VARIANTS",
@@ -145,6 +146,9 @@ def lib() -> ctypes.CDLL:
     L.hipgemm_select_variant.restype = ci
     L.hipgemm_split_columns.argtypes = [ci, ci, ci]
     L.hipgemm_split_columns.restype = ci
+    L.hipgemm_auto_tile.argtypes = [ci, ci, ci, ctypes.POINTER(ci),
+                                    ctypes.POINTER(ci)]
+    L.hipgemm_auto_tile.restype = ci
     L.hipgemm_gemm_workspace_size.argtypes = [ctypes.c_void_p]
     L.hipgemm_gemm_workspace_size.restype = ctypes.c_size_t
     L.hipgemm_variant_name.argtypes = [ci]
@@ -259,6 +263,16 @@ def split_columns(M: int, N: int, K: int) -> int:
     """Columns of C that AUTO runs on the 4-wave schedule when it splits C
     between the 4-wave and 128 x 128 schedules; 0 when it does not."""
     return int(lib().hipgemm_split_columns(M, N, K))
+
+
+def auto_tile(M: int, N: int, K: int):
+    """(rows, columns) of the tile AUTO runs 8-bit operands on where it is
+    another than select_variant's schedule has (hipgemm_auto_tile); else
+    None."""
+    bm, bn = ctypes.c_int(), ctypes.c_int()
+    if not lib().hipgemm_auto_tile(M, N, K, ctypes.byref(bm), ctypes.byref(bn)):
+        return None
+    return bm.value, bn.value
 
 
 def variant_name(v: int) -> Optional[str]:

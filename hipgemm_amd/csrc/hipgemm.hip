@@ -133,7 +133,8 @@ hipError_t launch_tiled(int variant, GemmArgs g, hk::Key key,
         break;
       }
       fn = !key.ext ? hk::four_wave_plain(16, key)
-           : key.out >= kOutF32          ? hk::four_wave_ext_wide(key)
+           : key.out == kOutF32          ? hk::four_wave_ext_f32(key)
+           : key.out == kOutF8           ? hk::four_wave_ext_f8(key)
            : key.out == HIPGEMM_OUT_F16 ? hk::four_wave_ext_f16(key)
                                         : hk::four_wave_ext_bf16(key);
       break;
@@ -141,6 +142,27 @@ hipError_t launch_tiled(int variant, GemmArgs g, hk::Key key,
   if (!fn) return hipErrorInvalidValue;  // no such instantiation
   void* args[] = {&g};
   return hipLaunchKernel(fn, dim3(grid), dim3(threads), args, 0, stream);
+}
+
+// The tile schedule on tile t of hk::kTiles; nullptr kernel where that tile
+// is not built for the call.  fp32 and e4m3 outputs: one store of four
+// elements per lane and block; 2-byte types: 16-byte stores.
+const void* tile_kernel(int t, const GemmArgs& g, hk::Key* key) {
+  key->vec = vec_ok(key->out, g.N, g.ldc, g.C, key->out >= kOutF32 ? 4 : 8);
+  return !key->ext            ? hk::tile_plain(t, *key)
+         : key->out < kOutF32 ? hk::tile_ext_narrow(t, *key)
+                              : hk::tile_ext_wide(t, *key);
+}
+
+hipError_t launch_tile(int t, const void* fn, GemmArgs g, hipStream_t stream) {
+  const int bm = hk::kTiles[t].bm, bn = hk::kTiles[t].bn;
+  const int tm = (g.M + bm - 1) / bm, tn = (g.N + bn - 1) / bn;
+  const int cus = cu_count();
+  g.group_m = default_group_m(tm, tn);
+  g.workers = tm * tn < cus ? tm * tn : cus;
+  void* args[] = {&g};
+  return hipLaunchKernel(fn, dim3(g.workers), dim3(CfgT128::kThreads), args, 0,
+                         stream);
 }
 
 // AUTO's column split (hipgemm_split_columns): g4 columns [0, n1) on the
@@ -374,6 +396,7 @@ hipError_t launch_strip(const GemmArgs& a, const StripPlan& p, void* ws,
                          args, 0, stream);
 }
 
+int ceil_div(int a, int b) { return (a + b - 1) / b; }
 int resolve_variant(int variant, int M, int N, int K);
 int fp4_variant(int variant, int M, int N, int Kb);
 
@@ -455,8 +478,6 @@ hipError_t launch_t128_split(GemmArgs g, const T128Plan& p, void* ws,
   return hipLaunchKernel(fn, dim3(tiles * 16), dim3(64), args, 0, stream);
 }
 
-int ceil_div(int a, int b) { return (a + b - 1) / b; }
-
 // AUTO's split of C's columns when the last round of 256 x 256 tiles would
 // leave most CUs idle (4000 x 5000: 320 tiles = 1.25 rounds): columns
 // [0, n1) on the 4-wave 16x16x128 schedule in whole rounds, the rest on the
@@ -477,6 +498,68 @@ int split_columns(int M, int N, int cus) {
   const double split = rounds + 0.6 * ceil_div(rest, cus);
   const double plain = ceil_div(tiles, cus);
   return split + 0.25 <= plain ? n1 : 0;
+}
+
+// Time model of AUTO's choice of tile above 128 rows (us on MI355X): a launch
+// of `tiles` tiles takes R = ceil(tiles / CUs) rounds, each `step` per 128-byte
+// K-step plus `busy` per step times the share of the CUs at work (shared
+// fetch paths, clock), plus a fixed time per round (fill of the first tile,
+// epilogue) and per launch.  Fitted to 298 shapes (129 to 8192 rows, N 1024 to
+// 28672, K 512 to 14336; half of them a grid of usual sizes, half random),
+// every tile timed on each: 5-9 % standard error per tile.
+struct TileCost {
+  int bm, bn;
+  double launch, round, step, busy;
+};
+constexpr TileCost kCost256{256, 256, 0.99, 6.86, 0.847, 0.370};
+constexpr TileCost kCost128{128, 128, 3.15, 1.23, 0.309, 0.149};
+constexpr TileCost kCostMid[hk::kNumTiles] = {{128, 256, 2.91, 2.57, 0.496, 0.248},
+                                              {192, 192, 2.92, 3.35, 0.507, 0.280},
+                                              {192, 128, 2.54, 2.15, 0.369, 0.213}};
+double tile_cost(const TileCost& c, int M, int N, int K, int cus) {
+  const int tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn);
+  const int rounds = ceil_div(tiles, cus);
+  return c.launch + c.round * rounds +
+         ceil_div(K, 128) * (c.step * rounds + c.busy * tiles / cus);
+}
+
+// AUTO's tile for 8-bit operands above 128 rows where it is neither the 256 x
+// 256 tile, the column split nor the K-split that hipgemm_select_variant and
+// hipgemm_split_columns name: an index of hk::kTiles, kTile128 (128 x 128, no
+// K-split), or kNoTile.  It has to come out 5 % below the cost of what those
+// name: over the 298 shapes AUTO is then 6 % faster on average (2048 x 4096 x
+// 4096 37.3 -> 26.5 us, 3072^3 28.7 -> 23.3, 1536 x 4096 x 4096 28.9 -> 20.0,
+// 1024 x 8192 x 4096 38 -> 30.5, 1024 x 1024 x 4096 19.2 -> 14.3), one shape
+// slower by more than 3 % (5.7 %); without the margin eight.
+constexpr int kNoTile = -1, kTile128 = -2;
+int pick_tile(int M, int N, int K, int cus) {
+  if (M <= CfgSkinny::kMaxM || K <= 0 || N <= 0) return kNoTile;
+  const int variant = hipgemm_select_variant(M, N, K);
+  const int n1 = split_columns(M, N, cus);
+  const T128Plan ks = plan_t128(M, N, K, cus);
+  const double c128 = tile_cost(kCost128, M, N, K, cus);
+  double now;
+  if (n1 > 0) {
+    now = 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus) +
+          0.91 * tile_cost(kCost128, M, N - n1, K, cus);
+  } else if (variant != HIPGEMM_VARIANT_TILE128) {
+    now = tile_cost(kCost256, M, N, K, cus);
+  } else if (ks.slices > 1) {
+    const double units = (double)ceil_div(M, 128) * ceil_div(N, 128) * ks.slices / cus;
+    now = 9.64 + ks.slice_steps * (0.207 + 0.073 * units) + 6.01 * units;
+  } else {
+    now = c128;
+  }
+  int best = kTile128;
+  double cost = c128;
+  for (int t = 0; t < hk::kNumTiles; ++t) {
+    const double c = tile_cost(kCostMid[t], M, N, K, cus);
+    if (c < cost) {
+      cost = c;
+      best = t;
+    }
+  }
+  return cost < 0.95 * now ? best : kNoTile;
 }
 
 bool valid_code(int v, int count) { return v >= 0 && v < count; }
@@ -598,6 +681,15 @@ hipError_t run_gemm(const hipgemm_gemm_desc& d, bool ws_given,
   key.act = d.activation;
   key.out = d.out_dtype;
   if (dry_run) return hipSuccess;
+  if (d.variant == HIPGEMM_VARIANT_AUTO && fmt < 4 && !mx) {
+    const int t = pick_tile(M, N, K, cu_count());
+    if (t == kTile128) return launch_tiled(HIPGEMM_VARIANT_TILE128, g, key, stream);
+    if (t >= 0) {
+      hk::Key k = key;
+      // Not built for every epilogue: else what follows.
+      if (const void* fn = tile_kernel(t, g, &k)) return launch_tile(t, fn, g, stream);
+    }
+  }
   // Whether a call that brings no workspace runs under stream capture: a
   // schedule that would split K then runs unsplit, as the stream-ordered
   // allocation of its partials would only be recorded into the caller's
@@ -829,7 +921,17 @@ int hipgemm_select_variant(int M, int N, int K) {
 
 int hipgemm_split_columns(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
-  return split_columns(M, N, cu_count());
+  const int cus = cu_count();
+  return pick_tile(M, N, K, cus) == kNoTile ? split_columns(M, N, cus) : 0;
+}
+
+int hipgemm_auto_tile(int M, int N, int K, int* bm, int* bn) {
+  if (!bm || !bn) return 0;
+  const int t = pick_tile(M, N, K, cu_count());
+  if (t == kNoTile) return 0;
+  *bm = t == kTile128 ? CfgT128::kBM : hk::kTiles[t].bm;
+  *bn = t == kTile128 ? CfgT128::kBN : hk::kTiles[t].bn;
+  return 1;
 }
 
 hipError_t hipgemm_fp8_gemm_bf16(const void* A, const void* B_T, void* C,

@@ -33,7 +33,8 @@ struct Key {
 const void* four_wave_plain(int mf, const Key& k);  // k4wave_plain.hip
 const void* four_wave_ext_bf16(const Key& k);       // k4wave_ext_bf16.hip
 const void* four_wave_ext_f16(const Key& k);        // k4wave_ext_f16.hip
-const void* four_wave_ext_wide(const Key& k);       // k4wave_ext_wide.hip
+const void* four_wave_ext_f32(const Key& k);        // k4wave_ext_f32.hip
+const void* four_wave_ext_f8(const Key& k);         // k4wave_ext_f8.hip
 const void* eight_wave_plain(const Key& k);         // k8wave_plain.hip
 const void* eight_wave_ext_bf16(const Key& k);      // k8wave_ext_bf16.hip
 const void* eight_wave_ext_f16(const Key& k);       // k8wave_ext_f16.hip
@@ -54,6 +55,9 @@ inline const void* tile128_ext(const Key& k) {
 const void* tile128_split(const Key& k);            // kt128_plain.hip
 const void* tile128_reduce(const Key& k);           // kt128_plain.hip
 const void* split_plain(const Key& k);              // ksplit_plain.hip
+const void* tile_plain(int tile, const Key& k);     // ktile_plain.hip
+const void* tile_ext_narrow(int tile, const Key& k);  // ktile_ext.hip
+const void* tile_ext_wide(int tile, const Key& k);    // ktile_ext_wide.hip
 // hipgemm_gemm_noalloc's static scratch array on the current device
 // (noalloc_scratch.hip): its address, looked up once per device (with that
 // device current); at that first lookup its counter region is cleared on
@@ -102,6 +106,22 @@ const void* sel4(int v, F&& f) {
     case 1: return f(ic<1>{});
     case 2: return f(ic<2>{});
     case 3: return f(ic<3>{});
+    default: return nullptr;
+  }
+}
+
+// The tiles between 128 x 128 and 256 x 256, in the order of kTiles.
+struct TileShape {
+  int bm, bn;
+};
+constexpr TileShape kTiles[] = {{128, 256}, {192, 192}, {192, 128}};
+constexpr int kNumTiles = 3;
+template <class F>
+const void* sel_tile(int t, F&& f) {
+  switch (t) {
+    case 0: return f(detail::CfgTile<kTiles[0].bm, kTiles[0].bn, 3>{});
+    case 1: return f(detail::CfgTile<kTiles[1].bm, kTiles[1].bn, 3>{});
+    case 2: return f(detail::CfgTile<kTiles[2].bm, kTiles[2].bn, 3>{});
     default: return nullptr;
   }
 }

@@ -372,6 +372,15 @@ int hipgemm_select_variant(int M, int N, int K);
  * M*N/65536 tiles of 256 x 256, fp8_4wave.hpp:357-377). */
 int hipgemm_split_columns(int M, int N, int K);
 
+/* AUTO's tile for 8-bit operands above 128 rows, where a tile between 128 x
+ * 128 and 256 x 256 (or 128 x 128 ones without a K-split) is estimated
+ * faster than the schedule hipgemm_select_variant names: returns 1 and the
+ * tile (bm x bn), or 0 when AUTO runs that schedule as it is.  Such calls run
+ * the 128 x 128 schedule's pipeline on 128 x 256, 192 x 192, 192 x 128 or 128
+ * x 128 tiles, in one launch without a workspace.  No reference counterpart
+ * (the reference has 256 x 256 tiles only). */
+int hipgemm_auto_tile(int M, int N, int K, int *bm, int *bn);
+
 /* Human-readable variant name, or NULL.  No reference counterpart. */
 const char *hipgemm_variant_name(int variant);
 

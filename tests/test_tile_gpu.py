@@ -1,0 +1,117 @@
+"""AUTO's tiles between 128 x 128 and 256 x 256 (hipgemm_auto_tile): where
+AUTO takes them, and their results against the oracle, bit for bit on ternary
+operands (every partial sum exact, in any order).
+
+Shapes end inside a tile in both directions, inside a K-step, or exactly on
+them, run one and several tiles per workgroup, and take 16-byte stores of C or
+not; every output type and epilogue option of the general entry point runs on
+every tile, with canaries around C.
+"""
+import numpy as np
+import pytest
+
+import hipgemm_amd as hg
+from oracle import pyoracle as po
+from util import say, to_dev
+
+TERN = {0: np.array([0xB8, 0x00, 0x38], np.uint8),
+        1: np.array([0xBC, 0x00, 0x3C], np.uint8)}
+ES = {po.OUT_BF16: 2, po.OUT_F16: 2, po.OUT_F32: 4, po.OUT_FP8: 1}
+NP = {4: np.uint32, 2: np.uint16, 1: np.uint8}
+
+# shape -> AUTO's tile on 256 CUs
+SHAPES = {
+    (144, 256, 2272): (128, 128),    # K-split plan, run unsplit
+    (190, 237, 2192): (128, 128),    # odd N: 2-byte stores
+    (4221, 1832, 16): (128, 128),    # two rounds, one K-step
+    (2055, 3640, 336): (128, 256),
+    (1201, 5891, 240): (128, 256),   # odd N
+    (4367, 4672, 144): (128, 256),   # several tiles per workgroup
+    (2304, 3840, 512): (192, 192),   # whole tiles and steps
+    (1865, 4391, 144): (192, 192),   # odd N
+    (4051, 4416, 432): (192, 192),   # several tiles per workgroup
+    (1237, 3280, 592): (192, 128),
+    (1537, 5392, 1040): (192, 128),  # several tiles per workgroup
+    (2119, 4149, 16): (192, 128),    # odd N, two rounds, one K-step
+    (2304, 2304, 1024): (192, 128),  # whole tiles and steps
+}
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_auto_tile(shape):
+    M, N, K = shape
+    assert hg.auto_tile(M, N, K) == SHAPES[shape]
+    assert hg.split_columns(M, N, K) == 0
+
+
+def test_auto_tile_keeps_other_choices():
+    """None up to 128 rows, where 256 x 256 tiles fill whole rounds, for the
+    documented column split, or without work."""
+    for M, N, K in [(128, 8192, 8192), (64, 4096, 4096), (8192, 8192, 8192),
+                    (4096, 4096, 4096), (8192, 28672, 8192), (4000, 5000, 3584),
+                    (256, 8192, 8192), (512, 512, 512), (300, 300, 0), (0, 64, 64)]:
+        assert hg.auto_tile(M, N, K) is None, (M, N, K)
+
+
+def run(torch, A, B, out, ldc, *, fb=0, act=0, sa=None, sr=None, sc=None, bias=None,
+        so=None):
+    M, K = A.shape
+    N = B.shape[0]
+    es = ES[out]
+    dev = {k: None if v is None else torch.from_numpy(
+        np.ascontiguousarray(v, np.float32).reshape(-1)).to("cuda")
+        for k, v in dict(sa=sa, sr=sr, sc=sc, bias=bias, so=so).items()}
+    ptr = {k: v.data_ptr() if v is not None else 0 for k, v in dev.items()}
+    a, b = to_dev(torch, A), to_dev(torch, B)
+    buf = torch.full(((M + 4) * ldc * es,), 0xA5, dtype=torch.uint8, device="cuda")
+    d = hg.GemmDesc(A=a.data_ptr(), B_T=b.data_ptr(), C=buf.data_ptr() + 2 * ldc * es,
+                    M=M, N=N, K=K, lda=K, ldb=K, ldc=ldc, b_format=fb,
+                    out_dtype=out, activation=act, scale_a=ptr["sa"],
+                    scale_rows=ptr["sr"], scale_cols=ptr["sc"], bias=ptr["bias"],
+                    scale_out=ptr["so"])
+    assert hg.gemm_desc_raw(d, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy().reshape(M + 4, ldc * es)
+    guard = (np.all(got[:2] == 0xA5) and np.all(got[M + 2:] == 0xA5) and
+             np.all(got[2:M + 2, N * es:] == 0xA5))
+    C = np.ascontiguousarray(got[2:M + 2, :N * es]).view(NP[es])
+    return C, guard
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_tile_bit_exact(gpu, oracle, shape):
+    M, N, K = shape
+    rng = np.random.default_rng(5)
+    for fb, pad in ((0, 0), (1, 8), (0, 3)):  # ldc = N + 3: 2-byte stores
+        say(f"case tile {SHAPES[shape]} M={M} N={N} K={K} fb={fb} ldc=N+{pad}")
+        A = TERN[0][rng.integers(0, 3, (M, K))]
+        B = TERN[fb][rng.integers(0, 3, (N, K))]
+        C, guard = run(gpu, A, B, po.OUT_BF16, N + pad, fb=fb, sa=[0.5])
+        want = oracle.gemm_ex(A, B, b_fmt=fb, scale_a=0.5)
+        assert guard, "write outside M x N"
+        assert np.array_equal(C, want), f"{int((C != want).sum())} of {C.size} differ"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("out", [po.OUT_BF16, po.OUT_F16, po.OUT_F32, po.OUT_FP8],
+                         ids=["bf16", "f16", "f32", "e4m3"])
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s[1] % 8 == 0],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_tile_epilogue(gpu, oracle, shape, out):
+    M, N, K = shape
+    rng = np.random.default_rng(6)
+    A, B = TERN[0][rng.integers(0, 3, (M, K))], TERN[1][rng.integers(0, 3, (N, K))]
+    sr = np.exp2(rng.integers(-3, 4, M)).astype(np.float32)
+    sc = np.exp2(rng.integers(-3, 4, N)).astype(np.float32)
+    bias = rng.uniform(-4, 4, N).astype(np.float32)
+    so = 0.25 if out == po.OUT_FP8 else None
+    for act in (po.ACT_NONE, po.ACT_RELU):
+        say(f"case tile {SHAPES[shape]} M={M} N={N} K={K} out={out} act={act}")
+        C, guard = run(gpu, A, B, out, N + 8, fb=1, act=act, sa=[0.5], sr=sr, sc=sc,
+                       bias=bias, so=None if so is None else [so])
+        want = oracle.gemm_ex(A, B, b_fmt=1, out=out, act=act, scale_a=0.5,
+                              scale_rows=sr, scale_cols=sc, bias=bias,
+                              scale_out=so or 1.0)
+        assert guard, "write outside M x N"
+        assert np.array_equal(C, want), f"{int((C != want).sum())} of {C.size} differ"
