@@ -137,6 +137,9 @@ def lib() -> ctypes.CDLL:
     L.hipgemm_mx_scales_bytes.restype = ctypes.c_size_t
     L.hipgemm_mx_pack_scales.argtypes = [vp, ci, ci, ci, vp, vp]
     L.hipgemm_mx_pack_scales.restype = ci
+    L.hipgemm_quantize_rows_e4m3.argtypes = [vp, ci, ci, ci, ctypes.c_longlong,
+                                             vp, vp, vp]
+    L.hipgemm_quantize_rows_e4m3.restype = ci
     L.hipgemm_workspace_size.argtypes = [ci, ci, ci, ci]
     L.hipgemm_workspace_size.restype = ctypes.c_size_t
     L.hipgemm_fp8_gemm_4wave_256x256x128.argtypes = [vp, vp, vp, ci, ci, ci,

@@ -997,6 +997,17 @@ hipError_t hipgemm_mx_pack_scales(const void* src, int rows, int K, int ld,
                      static_cast<uint8_t*>(dst), stream);
 }
 
+hipError_t hipgemm_quantize_rows_e4m3(const void* x, int type, int M, int K,
+                                      long long ldx, void* q, float* s,
+                                      hipStream_t stream) {
+  if (M < 0 || K < 0 || !valid_code(type, 3)) return hipErrorInvalidValue;
+  if (M == 0 || K == 0) return hipSuccess;
+  const int es = type == HIPGEMM_IN_F32 ? 4 : 2;
+  if (!x || !q || !s || ldx < K || !aligned(x, es) || !aligned(s, 4))
+    return hipErrorInvalidValue;
+  return hk::quantize_rows(x, type, M, K, ldx, q, s, stream);
+}
+
 size_t hipgemm_gemm_workspace_size(const hipgemm_gemm_desc* d) {
   if (!d || d->size != sizeof(hipgemm_gemm_desc) || d->M <= 0 || d->N <= 0 ||
       d->K <= 0)

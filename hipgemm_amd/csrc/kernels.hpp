@@ -65,6 +65,9 @@ const void* tile_ext_wide(int tile, const Key& k);    // ktile_ext_wide.hip
 // failure.
 void* noalloc_scratch(hipStream_t stream, hipError_t* err);
 // Packs [rows][ceil(K/32)] E8M0 scales (row stride ld) into MxArgs' layout.
+// Per-row e4m3 quantisation (kquant.hip); type: HIPGEMM_IN_*.
+hipError_t quantize_rows(const void* x, int type, int M, int K, long long ldx,
+                         void* q, float* s, hipStream_t stream);
 hipError_t mx_pack(const uint8_t* src, int rows, int K, int ld, uint8_t* dst,
                    hipStream_t stream);
 

@@ -41,6 +41,7 @@ from typing import Optional
 import torch
 
 from . import ACTIVATIONS, HipGemmError, fp8_gemm_bf16, fp8_gemm_bf16_rowcol
+from . import _check, lib
 from . import gemm as _gemm
 
 __all__ = ["fp8_gemm", "fp8_gemm_rowcol", "gemm", "Fp8Linear",
@@ -134,10 +135,53 @@ def _check_shapes(a, b_t):
                            f"{tuple(a.shape)} and {tuple(b_t.shape)}")
 
 
+# Input types of hipgemm_quantize_rows_e4m3.
+_QUANT_TYPES = {torch.float32: 0, torch.bfloat16: 1, torch.float16: 2}
+
+
+def _plain_eager(x: torch.Tensor) -> bool:
+    """x is an ordinary tensor on the current GPU and nothing watches the
+    operations on it: no autograd graph to record (reverse or forward), no
+    transform, trace, compilation or dispatch mode.  Everything else takes the
+    tensor operations, which all of those see."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and x.is_cuda
+            and x.layout is torch.strided and not x.is_neg()
+            and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch.compiler.is_compiling()
+            and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0
+            and torch._C._len_torch_function_stack() == 0
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0
+            and x.device.index == torch.cuda.current_device())
+
+
 def quantize_rows(x: torch.Tensor):
     """Per-row e4m3 quantisation: returns (q, s) with q = x / s rounded to
     e4m3 (saturated to +-448) and s = amax(|row|) / 448 (float32, one per
-    row; rows of zeros get s = 1).  x ~= q * s[:, None]."""
+    row; rows of zeros get s = 1).  x ~= q * s[:, None].
+
+    Rows of float32, bfloat16 or float16 on the GPU go through one kernel
+    (hipgemm_quantize_rows_e4m3), with the same results bit for bit; under
+    autograd, a transform or a trace, on the CPU and for other layouts these
+    are tensor operations."""
+    if (_plain_eager(x) and x.dim() == 2 and x.dtype in _QUANT_TYPES
+            and x.numel() > 0 and x.stride(1) == 1
+            and x.stride(0) >= x.shape[1]
+            and x.shape[0] < 2 ** 31 and x.shape[1] < 2 ** 31):
+        M, K = x.shape
+        q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
+        s = torch.empty((M,), dtype=torch.float32, device=x.device)
+        _check(int(lib().hipgemm_quantize_rows_e4m3(
+            x.data_ptr(), _QUANT_TYPES[x.dtype], M, K, x.stride(0), q.data_ptr(),
+            s.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream or None)),
+            "hipgemm_quantize_rows_e4m3")
+        return q, s
+    return _quantize_rows_ops(x)
+
+
+def _quantize_rows_ops(x: torch.Tensor):
+    """quantize_rows as tensor operations."""
     xf = x.float()
     amax = xf.abs().amax(dim=1)
     s = torch.where(amax > 0, amax / E4M3_MAX, torch.ones_like(amax))

@@ -339,6 +339,20 @@ size_t hipgemm_mx_scales_bytes(int rows, int K);
 hipError_t hipgemm_mx_pack_scales(const void *src, int rows, int K, int ld,
                                   void *dst, hipStream_t stream);
 
+/*
+ * Per-row e4m3 quantisation of x (M x K, device, row stride ldx elements, of
+ * type HIPGEMM_IN_*): s[m] = max |x[m, :]| times fp32(1 / 448), or 1 where that
+ * maximum is 0 or NaN; q[m, k] (M x K packed bytes) = e4m3 of x[m, k] / s[m]
+ * clamped to +-448, round to nearest even, NaN kept.  So x ~= q * s[m], and q, s
+ * are hipgemm_gemm's A and scale_rows.  x aligned to its type, s to 4 bytes,
+ * ldx >= K; M == 0 or K == 0 is a no-op.  One launch on `stream`.
+ * No reference counterpart (the reference takes e4m3 operands as they are).
+ */
+enum { HIPGEMM_IN_F32 = 0, HIPGEMM_IN_BF16 = 1, HIPGEMM_IN_F16 = 2 };
+hipError_t hipgemm_quantize_rows_e4m3(const void *x, int type, int M, int K,
+                                      long long ldx, void *q, float *s,
+                                      hipStream_t stream);
+
 /* Workspace bytes hipgemm_fp8_gemm_bf16_ws needs for this shape and variant
  * on the current device (0: none).  No GPU work.  No reference counterpart. */
 size_t hipgemm_workspace_size(int M, int N, int K, int variant);
