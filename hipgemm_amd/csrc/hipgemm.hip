@@ -88,6 +88,13 @@ bool line_ok(int out, int ldc, const void* C) {
   return out_bytes(out) == 2 && ldc % 64 == 0 && aligned(C, 128);
 }
 
+// K-slices of 64-column tiles (plan_narrow below): tile of hk::kNarrow.
+struct NarrowPlan {
+  int tile = -1, slices = 1, slice_steps = 0;
+  size_t ws_bytes = 0;
+  double cost = 1e9;  // us, the time model's
+};
+
 // The tiled schedules (4-wave, 8-wave) on a persistent grid: one workgroup
 // per CU at most (their 160 KiB of LDS allows no more), each walking tiles
 // w, w + grid, ...  `key.vec` is set here: 16-byte epilogue stores need
@@ -160,6 +167,36 @@ hipError_t launch_tile(int t, const void* fn, GemmArgs g, hipStream_t stream) {
   const int cus = cu_count();
   g.group_m = default_group_m(tm, tn);
   g.workers = tm * tn < cus ? tm * tn : cus;
+  void* args[] = {&g};
+  return hipLaunchKernel(fn, dim3(g.workers), dim3(CfgT128::kThreads), args, 0,
+                         stream);
+}
+
+// 64-column tiles on plan p; nullptr where they are not built for the call.
+const void* narrow_kernel(const NarrowPlan& p, const GemmArgs& g, hk::Key* key) {
+  const int mode = p.slices > 1 ? hk::kNarrowSplit
+                   : g.M <= hk::kNarrow[p.tile].bm ? hk::kNarrowOnce
+                                                   : hk::kNarrowWhole;
+  key->vec = vec_ok(key->out, g.N, g.ldc, g.C, key->out >= kOutF32 ? 4 : 8);
+  return !key->ext            ? hk::narrow_plain(p.tile, mode, *key)
+         : key->out < kOutF32 ? hk::narrow_ext(p.tile, mode, *key)
+                              : hk::narrow_ext_wide(p.tile, mode, *key);
+}
+
+hipError_t launch_narrow(const NarrowPlan& p, const void* fn, GemmArgs g, void* ws,
+                         hipStream_t stream) {
+  const int bm = hk::kNarrow[p.tile].bm, bn = hk::kNarrow[p.tile].bn;
+  const int tm = (g.M + bm - 1) / bm, tn = (g.N + bn - 1) / bn;
+  const int units = tm * tn * p.slices, cus = cu_count();
+  g.group_m = default_group_m(tm, tn);
+  g.workers = units < cus ? units : cus;
+  if (p.slices > 1) {
+    g.split.slices = p.slices;
+    g.split.slice_steps = p.slice_steps;
+    g.split.arrivals = static_cast<int*>(ws);
+    g.split.partial =
+        reinterpret_cast<float*>(static_cast<char*>(ws) + HIPGEMM_WS_COUNTER_BYTES);
+  }
   void* args[] = {&g};
   return hipLaunchKernel(fn, dim3(g.workers), dim3(CfgT128::kThreads), args, 0,
                          stream);
@@ -523,43 +560,160 @@ double tile_cost(const TileCost& c, int M, int N, int K, int cus) {
          ceil_div(K, 128) * (c.step * rounds + c.busy * tiles / cus);
 }
 
-// AUTO's tile for 8-bit operands above 128 rows where it is neither the 256 x
-// 256 tile, the column split nor the K-split that hipgemm_select_variant and
-// hipgemm_split_columns name: an index of hk::kTiles, kTile128 (128 x 128, no
-// K-split), or kNoTile.  It has to come out 5 % below the cost of what those
-// name: over the 298 shapes AUTO is then 6 % faster on average (2048 x 4096 x
-// 4096 37.3 -> 26.5 us, 3072^3 28.7 -> 23.3, 1536 x 4096 x 4096 28.9 -> 20.0,
-// 1024 x 8192 x 4096 38 -> 30.5, 1024 x 1024 x 4096 19.2 -> 14.3), one shape
-// slower by more than 3 % (5.7 %); without the margin eight.
-constexpr int kNoTile = -1, kTile128 = -2;
-int pick_tile(int M, int N, int K, int cus) {
-  if (M <= CfgSkinny::kMaxM || K <= 0 || N <= 0) return kNoTile;
+// Cost of what hipgemm_select_variant and hipgemm_split_columns name for 33
+// rows and more (the same model; the strip's per step the bytes of its columns
+// and of A's row blocks; 5-7 % standard error on 146 and 135 shapes up to 128
+// rows).
+double named_cost(int M, int N, int K, int cus) {
   const int variant = hipgemm_select_variant(M, N, K);
-  const int n1 = split_columns(M, N, cus);
-  const T128Plan ks = plan_t128(M, N, K, cus);
-  const double c128 = tile_cost(kCost128, M, N, K, cus);
-  double now;
-  if (n1 > 0) {
-    now = 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus) +
-          0.91 * tile_cost(kCost128, M, N - n1, K, cus);
-  } else if (variant != HIPGEMM_VARIANT_TILE128) {
-    now = tile_cost(kCost256, M, N, K, cus);
-  } else if (ks.slices > 1) {
-    const double units = (double)ceil_div(M, 128) * ceil_div(N, 128) * ks.slices / cus;
-    now = 9.64 + ks.slice_steps * (0.207 + 0.073 * units) + 6.01 * units;
-  } else {
-    now = c128;
+  if (variant == HIPGEMM_VARIANT_STRIP) {
+    const StripPlan p = plan_strip(M, N, K, strip_knb(M, N, K));
+    const double w = p.knb / 2.0, area = p.kmb * p.knb / 8.0;
+    const int rounds = ceil_div(p.tiles_n * p.slices, cus);
+    return 3.54 + p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) + 1.10 * area +
+           (p.slices > 1 ? 2.02 + 0.189 * p.slices * area : 0.0);
   }
-  int best = kTile128;
-  double cost = c128;
-  for (int t = 0; t < hk::kNumTiles; ++t) {
-    const double c = tile_cost(kCostMid[t], M, N, K, cus);
-    if (c < cost) {
-      cost = c;
-      best = t;
+  // The split-K schedule: never ahead of 64-column tiles where it is named.
+  if (variant == HIPGEMM_VARIANT_SKINNY) return 1e9;
+  const int n1 = split_columns(M, N, cus);
+  if (n1 > 0)
+    return 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus) +
+           0.91 * tile_cost(kCost128, M, N - n1, K, cus);
+  if (variant != HIPGEMM_VARIANT_TILE128) return tile_cost(kCost256, M, N, K, cus);
+  const T128Plan ks = plan_t128(M, N, K, cus);
+  const double units = (double)ceil_div(M, 128) * ceil_div(N, 128) * ks.slices / cus;
+  if (M <= CfgSkinny::kMaxM) {
+    const double c = 3.81 + ks.slice_steps * (0.375 * ceil_div((int)(units * cus), cus) + 0.326 * units) +
+                     (ks.slices > 1 ? 3.36 + 3.82 * units + 0.07 * (ks.slices - 1) : 0.0);
+    const double hbm = 3.0 + (double)N * K / 5.4e6;  // B_T at 5.4 TB/s
+    return c > hbm ? c : hbm;
+  }
+  return ks.slices > 1 ? 9.64 + ks.slice_steps * (0.207 + 0.073 * units) + 6.01 * units
+                       : tile_cost(kCost128, M, N, K, cus);
+}
+
+// 64-column tiles (hk::kNarrow) in `slices` K-slices: a stream over B_T for
+// few rows.  Why they are ahead: a CU's fetch path carries about 60 GB/s of
+// such streams whatever is in flight (a DMA-only loop), so that A's rows, read
+// again by every column of tiles, count as much as B_T's; and with K-slices
+// half the fp32 partials of 128 x 128 tiles go out and come back, the last
+// arrivals that sum them spread over twice the CUs.  Us, before -> after: 128 x
+// 8192 x 8192 (2 slices) 22.5 -> 20.9, 128 x 14336 x 4096 23.4 -> 17.7, 128 x
+// 8192 x 2048 13.6 -> 8.2, 64 x 8192 x 8192 (64 x 64, 2 slices) 21.0 -> 16.3,
+// 64 x 14336 x 4096 17.9 -> 13.8, 256 x 4096 x 4096 (64 x 64) 19.0 -> 11.7.
+// Model as above plus the slices' terms, fitted apart up to 128 rows and above
+// (7 % standard error over 440 and 320 shapes, every plan timed).
+struct NarrowCost {
+  double launch, round, step, busy, split, units, slice;
+};
+constexpr NarrowCost kNarrowFew[hk::kNumNarrow] = {
+    {2.84, 1.46, 0.265, 0.092, 0.06, 3.39, 0.633},
+    {2.98, 0.97, 0.200, 0.088, 0.00, 1.67, 0.541}};
+constexpr NarrowCost kNarrowMany[hk::kNumNarrow] = {
+    {3.04, 0.89, 0.236, 0.119, 0.68, 2.77, 0.787},
+    {2.92, 0.82, 0.156, 0.075, 0.96, 1.04, 0.607}};
+// The cheapest plan: K-slices of at least 8 steps, at most one workgroup per
+// CU, within max_ws bytes of workspace.  hbm: bytes per us that a stream of B_T
+// under one row of tiles reaches.
+NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm) {
+  NarrowPlan best;
+  const int steps = ceil_div(K, 128);
+  for (int t = 0; t < hk::kNumNarrow; ++t) {
+    const bool few = M <= CfgSkinny::kMaxM;
+    const NarrowCost& c = few ? kNarrowFew[t] : kNarrowMany[t];
+    const int tiles = ceil_div(M, hk::kNarrow[t].bm) * ceil_div(N, hk::kNarrow[t].bn);
+    for (int s = 1; s <= 8; ++s) {
+      if (s > 1 && (tiles * s > cus || 8 * s > steps)) break;
+      NarrowPlan p;
+      p.tile = t;
+      p.slice_steps = s > 1 ? (ceil_div(steps, s) + 1) & ~1 : steps;
+      p.slices = ceil_div(steps, p.slice_steps);
+      const int units = tiles * p.slices, rounds = ceil_div(units, cus);
+      const double share = (double)units / cus;
+      p.cost = c.launch + c.round * rounds + p.slice_steps * (c.step * rounds + c.busy * share);
+      if (p.slices > 1) {
+        p.cost += c.split + c.units * share + c.slice * (p.slices - 1);
+        p.ws_bytes = kWsCounterBytes +
+                     (size_t)units * hk::kNarrow[t].bm * hk::kNarrow[t].bn * sizeof(float);
+        if (p.ws_bytes > max_ws || 4 * tiles > kWsMaxCounters) continue;
+      }
+      if (few && p.cost < 3.0 + (double)N * K / hbm) p.cost = 3.0 + (double)N * K / hbm;
+      if (p.cost < best.cost) best = p;
     }
   }
-  return cost < 0.95 * now ? best : kNoTile;
+  return best;
+}
+
+// AUTO's tile for 8-bit operands above 32 rows where it is another than what
+// hipgemm_select_variant and hipgemm_split_columns name: an index of
+// hk::kTiles, kTile128 (128 x 128, no K-split), kTileNarrow (`narrow`), or
+// kNoTile.
+//  * Above 128 rows the tiles between 128 x 128 and 256 x 256, 5 % below the
+//    named cost: over 298 shapes 6 % faster on average (2048 x 4096 x 4096 37.3
+//    -> 26.5 us, 3072^3 28.7 -> 23.3, 1536 x 4096 x 4096 28.9 -> 20.0, 1024 x
+//    8192 x 4096 38 -> 30.5, 1024 x 1024 x 4096 19.2 -> 14.3), one slower by
+//    more than 3 % (5.7 %); without the margin eight.
+//  * 64-column tiles up to 1024 rows: 6 % below from 33 to 128 rows (277
+//    shapes: 17 % faster on average, three slower by more than 3 %, 10 % at
+//    worst), 10 % below a K-split of 128 x 128 tiles above (its cost is the
+//    least certain; 320 shapes up to 1024 rows: 11 % faster on average, 13 %
+//    slower at worst), else 5 %.  Up to 32 rows the strip, which reads A into
+//    registers, stays ahead.
+// max_ws: workspace bytes that K-slices may take (0: none).
+constexpr int kNoTile = -1, kTile128 = -2, kTileNarrow = -3;
+int pick_tile(int M, int N, int K, int cus, size_t max_ws, NarrowPlan* narrow) {
+  if (M <= 32 || K <= 0 || N <= 0) return kNoTile;
+  const double named = named_cost(M, N, K, cus);
+  int best = kNoTile;
+  double cost = named;
+  if (M > CfgSkinny::kMaxM) {
+    const double c128 = tile_cost(kCost128, M, N, K, cus);
+    if (c128 < 0.95 * named) {
+      best = kTile128;
+      cost = c128;
+    }
+    for (int t = 0; t < hk::kNumTiles; ++t) {
+      const double c = tile_cost(kCostMid[t], M, N, K, cus);
+      if (c < 0.95 * named && c < cost) {
+        cost = c;
+        best = t;
+      }
+    }
+    if (M > 1024) return best;
+  }
+  const bool t128 = hipgemm_select_variant(M, N, K) == HIPGEMM_VARIANT_TILE128;
+  const bool ksplit = M > CfgSkinny::kMaxM && best == kNoTile && t128 &&
+                      plan_t128(M, N, K, cus).slices > 1;
+  // 5.3 TB/s measured; 4.6 against 128 x 128 tiles, whose own stream is as
+  // fast there (over 100 MB of B_T).
+  *narrow = plan_narrow(M, N, K, cus, max_ws, t128 ? 4.6e6 : 5.3e6);
+  const double margin = M <= CfgSkinny::kMaxM ? 0.94 : ksplit ? 0.90 : 0.95;
+  return narrow->cost < margin * cost ? kTileNarrow : best;
+}
+
+// Workspace of the schedule `variant` (a resolved one) for 8-bit operands.
+size_t variant_ws(int M, int N, int K, int variant) {
+  if (variant == HIPGEMM_VARIANT_TILE128) return plan_t128(M, N, K, cu_count()).ws_bytes;
+  if (variant == HIPGEMM_VARIANT_STRIP)
+    return M > CfgStrip::kMaxM ? 0 : plan_strip(M, N, K, strip_knb(M, N, K)).ws_bytes;
+  if (variant == HIPGEMM_VARIANT_SKINNY)
+    return M > CfgSkinny::kMaxM ? 0 : plan_skinny(M, N, K).ws_bytes;
+  return 0;
+}
+// What AUTO's 64-column K-slices may take: up to 128 rows what they need
+// (hipgemm_workspace_size covers it, at most 8 MiB on 256 CUs), above no more
+// than the named schedule's workspace.
+size_t narrow_max_ws(int M, int N, int K, int variant) {
+  return M <= CfgSkinny::kMaxM ? (size_t)HIPGEMM_NOALLOC_SCRATCH_BYTES
+                               : variant_ws(M, N, K, variant);
+}
+
+// Workspace of an AUTO call that names `variant` and picked t (narrow).
+size_t auto_ws(int M, int N, int K, int variant, int t, const NarrowPlan& narrow) {
+  const size_t need = variant_ws(M, N, K, variant);
+  return t == kTileNarrow && M <= CfgSkinny::kMaxM && narrow.ws_bytes > need
+             ? narrow.ws_bytes
+             : need;
 }
 
 bool valid_code(int v, int count) { return v >= 0 && v < count; }
@@ -681,13 +835,27 @@ hipError_t run_gemm(const hipgemm_gemm_desc& d, bool ws_given,
   key.act = d.activation;
   key.out = d.out_dtype;
   if (dry_run) return hipSuccess;
-  if (d.variant == HIPGEMM_VARIANT_AUTO && fmt < 4 && !mx) {
-    const int t = pick_tile(M, N, K, cu_count());
-    if (t == kTile128) return launch_tiled(HIPGEMM_VARIANT_TILE128, g, key, stream);
-    if (t >= 0) {
-      hk::Key k = key;
-      // Not built for every epilogue: else what follows.
-      if (const void* fn = tile_kernel(t, g, &k)) return launch_tile(t, fn, g, stream);
+  if (d.variant == HIPGEMM_VARIANT_AUTO && fmt < 4 && !mx && K > 0) {
+    NarrowPlan np;
+    const size_t max_ws = ws_given ? narrow_max_ws(M, N, K, variant) : 0;
+    int t = pick_tile(M, N, K, cu_count(), max_ws, &np);
+    // A workspace too small for what hipgemm_workspace_size names is refused
+    // whichever schedule runs.
+    if (ws_given && ws_bytes < auto_ws(M, N, K, variant, t, np)) return hipErrorInvalidValue;
+    // fp32 and e4m3 outputs are not built for the 64-column K-slices.
+    if (t == kTileNarrow && np.slices > 1 && key.out >= kOutF32)
+      t = pick_tile(M, N, K, cu_count(), 0, &np);
+    // The tiles are not built for every epilogue: else what follows.
+    hk::Key k = key;
+    const void* fn = nullptr;
+    if (t == kTileNarrow) {
+      fn = narrow_kernel(np, g, &k);
+      if (fn) return launch_narrow(np, fn, g, ws, stream);
+    } else if (t == kTile128) {
+      return launch_tiled(HIPGEMM_VARIANT_TILE128, g, key, stream);
+    } else if (t >= 0) {
+      fn = tile_kernel(t, g, &k);
+      if (fn) return launch_tile(t, fn, g, stream);
     }
   }
   // Whether a call that brings no workspace runs under stream capture: a
@@ -922,15 +1090,22 @@ int hipgemm_select_variant(int M, int N, int K) {
 int hipgemm_split_columns(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int cus = cu_count();
-  return pick_tile(M, N, K, cus) == kNoTile ? split_columns(M, N, cus) : 0;
+  NarrowPlan np;
+  return pick_tile(M, N, K, cus, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
 }
 
 int hipgemm_auto_tile(int M, int N, int K, int* bm, int* bn) {
   if (!bm || !bn) return 0;
-  const int t = pick_tile(M, N, K, cu_count());
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  NarrowPlan np;
+  const int t = pick_tile(M, N, K, cu_count(),
+                          narrow_max_ws(M, N, K, hipgemm_select_variant(M, N, K)), &np);
   if (t == kNoTile) return 0;
-  *bm = t == kTile128 ? CfgT128::kBM : hk::kTiles[t].bm;
-  *bn = t == kTile128 ? CfgT128::kBN : hk::kTiles[t].bn;
+  const hk::TileShape s = t == kTileNarrow ? hk::kNarrow[np.tile]
+                          : t == kTile128  ? hk::TileShape{CfgT128::kBM, CfgT128::kBN}
+                                           : hk::kTiles[t];
+  *bm = s.bm;
+  *bn = s.bn;
   return 1;
 }
 
@@ -1061,13 +1236,13 @@ hipError_t hipgemm_gemm_noalloc(const hipgemm_gemm_desc* desc,
 
 size_t hipgemm_workspace_size(int M, int N, int K, int variant) {
   if (M <= 0 || N <= 0 || K < 0) return 0;
-  const int v = resolve_variant(variant, M, N, K);
-  if (v == HIPGEMM_VARIANT_TILE128) return plan_t128(M, N, K, cu_count()).ws_bytes;
-  if (v == HIPGEMM_VARIANT_STRIP)
-    return M > CfgStrip::kMaxM ? 0 : plan_strip(M, N, K, strip_knb(M, N, K)).ws_bytes;
-  if (v != HIPGEMM_VARIANT_SKINNY) return 0;
-  if (M > CfgSkinny::kMaxM) return 0;
-  return plan_skinny(M, N, K).ws_bytes;
+  const int named = hipgemm_select_variant(M, N, K);
+  const int v = variant == HIPGEMM_VARIANT_AUTO ? named : variant;
+  if (v != named || K == 0) return variant_ws(M, N, K, v);
+  // The schedule AUTO names covers AUTO's 64-column K-slices too.
+  NarrowPlan np;
+  const int t = pick_tile(M, N, K, cu_count(), narrow_max_ws(M, N, K, v), &np);
+  return auto_ws(M, N, K, v, t, np);
 }
 
 hipError_t hipgemm_fp8_gemm_4wave_256x256x128(const void* A, const void* B_T,

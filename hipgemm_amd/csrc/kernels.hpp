@@ -58,6 +58,12 @@ const void* split_plain(const Key& k);              // ksplit_plain.hip
 const void* tile_plain(int tile, const Key& k);     // ktile_plain.hip
 const void* tile_ext_narrow(int tile, const Key& k);  // ktile_ext.hip
 const void* tile_ext_wide(int tile, const Key& k);    // ktile_ext_wide.hip
+// 64-column tiles.  mode: one K-slice, one with B_T read once (kNt), or
+// K-slices.
+enum { kNarrowWhole = 0, kNarrowOnce = 1, kNarrowSplit = 2 };
+const void* narrow_plain(int tile, int mode, const Key& k);       // knarrow_plain.hip
+const void* narrow_ext(int tile, int mode, const Key& k);         // knarrow_ext.hip
+const void* narrow_ext_wide(int tile, int mode, const Key& k);    // knarrow_ext_wide.hip
 // hipgemm_gemm_noalloc's static scratch array on the current device
 // (noalloc_scratch.hip): its address, looked up once per device (with that
 // device current); at that first lookup its counter region is cleared on
@@ -113,12 +119,13 @@ const void* sel4(int v, F&& f) {
   }
 }
 
-// The tiles between 128 x 128 and 256 x 256, in the order of kTiles.
+// The tiles between 128 x 128 and 256 x 256, and the 64-column ones.
 struct TileShape {
   int bm, bn;
 };
-constexpr TileShape kTiles[] = {{128, 256}, {192, 192}, {192, 128}};
-constexpr int kNumTiles = 3;
+constexpr int kNumTiles = 3, kNumNarrow = 2;
+constexpr TileShape kTiles[kNumTiles] = {{128, 256}, {192, 192}, {192, 128}};
+constexpr TileShape kNarrow[kNumNarrow] = {{128, 64}, {64, 64}};
 template <class F>
 const void* sel_tile(int t, F&& f) {
   switch (t) {
@@ -127,6 +134,19 @@ const void* sel_tile(int t, F&& f) {
     case 2: return f(detail::CfgTile<kTiles[2].bm, kTiles[2].bn, 3>{});
     default: return nullptr;
   }
+}
+// Six LDS stages (144 and 96 KiB): these tiles are streams over B_T.
+template <class F>
+const void* sel_narrow(int t, F&& f) {
+  switch (t) {
+    case 0: return f(detail::CfgTile<kNarrow[0].bm, kNarrow[0].bn, 6>{});
+    case 1: return f(detail::CfgTile<kNarrow[1].bm, kNarrow[1].bn, 6>{});
+    default: return nullptr;
+  }
+}
+template <class F>
+const void* sel3(int v, F&& f) {
+  return v == 0 ? f(ic<0>{}) : v == 1 ? f(ic<1>{}) : v == 2 ? f(ic<2>{}) : nullptr;
 }
 
 }  // namespace kernels

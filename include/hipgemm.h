@@ -386,13 +386,16 @@ int hipgemm_select_variant(int M, int N, int K);
  * M*N/65536 tiles of 256 x 256, fp8_4wave.hpp:357-377). */
 int hipgemm_split_columns(int M, int N, int K);
 
-/* AUTO's tile for 8-bit operands above 128 rows, where a tile between 128 x
- * 128 and 256 x 256 (or 128 x 128 ones without a K-split) is estimated
- * faster than the schedule hipgemm_select_variant names: returns 1 and the
- * tile (bm x bn), or 0 when AUTO runs that schedule as it is.  Such calls run
- * the 128 x 128 schedule's pipeline on 128 x 256, 192 x 192, 192 x 128 or 128
- * x 128 tiles, in one launch without a workspace.  No reference counterpart
- * (the reference has 256 x 256 tiles only). */
+/* AUTO's tile for 8-bit operands above 32 rows, where another tile is
+ * estimated faster than the schedule hipgemm_select_variant names: returns 1
+ * and the tile (bm x bn), or 0 when AUTO runs that schedule as it is.  Such
+ * calls run the 128 x 128 schedule's pipeline in one launch on 128 x 256, 192
+ * x 192, 192 x 128 or 128 x 128 tiles (above 128 rows, no workspace) or, up to
+ * 1024 rows, on 128 x 64 or 64 x 64 tiles -- those in K-slices where that is
+ * faster and the call brings the workspace hipgemm_workspace_size names for
+ * AUTO (or runs hipgemm_gemm_noalloc), the last slice to arrive at a part of a
+ * tile summing it.  No reference counterpart (the reference has 256 x 256
+ * tiles only). */
 int hipgemm_auto_tile(int M, int N, int K, int *bm, int *bn);
 
 /* Human-readable variant name, or NULL.  No reference counterpart. */

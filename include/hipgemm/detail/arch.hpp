@@ -86,6 +86,15 @@ __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rsrc,
       (int)voffset, (int)soffset, 0, 0);
 }
 
+// dma16 with the non-temporal hint, for data one workgroup reads once.
+__device__ __forceinline__ void dma16_nt(__amdgpu_buffer_rsrc_t rsrc,
+                                         lds_u8* lds_wave_base, uint32_t voffset,
+                                         uint32_t soffset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      rsrc, (__attribute__((address_space(3))) void*)lds_wave_base, 16,
+      (int)voffset, (int)soffset, 0, kStoreC);
+}
+
 // 4 bytes per lane, global (rsrc + voffset) -> LDS (lds_wave_base + 4 * lane);
 // each lane's range check covers exactly its own 4 bytes.
 __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t rsrc,

@@ -71,6 +71,11 @@
 // own; both add +0 + slice 0 + slice 1 + ... in fp32, so their outputs are the
 // same.
 //
+// kNt: B_T's DMA carry the non-temporal hint, for one row of tiles, where each
+// B_T line is read by one workgroup (64 x 14336 x 4096 on 64 x 64 tiles 14.9 ->
+// 13.8 us, 128 x 14336 x 4096 18.5 -> 17.7; with K-slices level to 10 %
+// slower).
+//
 // kMx: MX block scales from g.mx (the packed layout of MxArgs; per-tensor
 // epilogue).  Each step also loads, two steps ahead, each operand's 16 scale
 // bytes of the lane into registers (one buffer load per operand).
@@ -101,18 +106,20 @@ struct CfgTile {
   static constexpr int kFA = kWM / 16, kFB = kWN / 16;  // 16-row fragments
   static constexpr int kAStage = kBM * kBK;
   static constexpr int kStage = kAStage + kBN * kBK;
-  static constexpr int kStoreStage = 16 * kWN * 2;  // 16 rows of C per wave
+  // Staging per wave: 16 rows of C, or kExt's vectors (1.5 KiB).
+  static constexpr int kRows16 = 16 * kWN * 2;
+  static constexpr int kStoreStage = kRows16 > 1536 ? kRows16 : 1536;
   static constexpr int kStoreBase = kStages * kStage;
-  // The staging areas also hold kExt's vectors (1.5 KiB per wave).
+  static constexpr int kPartial = BM * BN * 4;  // a K-slice's fp32 tile
   static constexpr int kLdsBytes = kStoreBase + 4 * kStoreStage;
   static constexpr int kDmaA = BM / 32, kDmaB = BN / 32;  // per wave per step
   static constexpr int kDma = kDmaA + kDmaB;
-  static_assert(kLdsBytes <= 160 * 1024 && kStoreStage >= 1536, "LDS");
+  static_assert(kLdsBytes <= 160 * 1024, "LDS");
 };
 
 template <class Cfg, bool kVec, bool kExt = false, int kFmt = 0,
           int kAct = kActNone, int kOut = kOutBf16, bool kSplit = false,
-          bool kMx = false>
+          bool kMx = false, bool kNt = false>
 __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
   constexpr int S = Cfg::kStages, FA = Cfg::kFA, FB = Cfg::kFB;
   constexpr int kDma = Cfg::kDma;           // DMA per wave per step
@@ -125,20 +132,20 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
   constexpr int kPieces = k6 ? 3 : 2;
   constexpr int kReads = kPieces * (FA + FB);
   // MFMA of a step issued after the next step's barrier (none, one and two
-  // measured within 1 %).
-  constexpr int kMfma = FA * FB, kTail = 1, kHead = kMfma - kTail;
+  // measured within 1 %; none where every MFMA is needed to carry its reads).
+  constexpr int kMfma = FA * FB;
+  constexpr int kTail = kReads <= 2 * (kMfma - 1) ? 1 : 0, kHead = kMfma - kTail;
   // Reads go one per MFMA, two for the first kReads - kHead of them.
   constexpr int kTwo = kReads > kHead ? kReads - kHead : 0;
   static_assert(kReads <= 2 * kHead && kDma <= kHead, "one DMA per MFMA");
-  static_assert(!(kSplit && kExt), "the split kernels take the plain epilogue");
   static_assert(!kMx || (!kExt && !k6), "MX: per-tensor epilogue, 8-bit and fp4");
-  static_assert((!kSplit && !kMx) || (Cfg::kBM == 128 && Cfg::kBN == 128),
-                "K-slices, MX: 128 x 128 tiles");
+  static_assert(!kMx || (Cfg::kBM == 128 && Cfg::kBN == 128),
+                "MX: 128 x 128 tiles");
   // Stores of C per wave per tile (16-byte path), or of a partial or of wide
   // outputs (one per block straight from the accumulators).
   constexpr int kStores = kSplit || (kExt && kOut >= kOutF32)
                               ? FA * FB
-                              : FA * (Cfg::kStoreStage / 1024);
+                              : FA * (Cfg::kRows16 / 1024);
   static_assert((S - 2) * kD + kStores < 64, "vmcnt range");
   const int lane = lane_id();
   const int wave = wave_id();
@@ -237,9 +244,11 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
     const bool is_a = n < Cfg::kDmaA;
     const int q = is_a ? n : n - Cfg::kDmaA;
     const uint32_t vo = is_a ? voff_a[q] : voff_b[q];
-    dma16(is_a ? s.a : s.b,
-          lds + dst + (is_a ? 0 : Cfg::kAStage) + (4 * q + wave) * 1024,
-          kEdge ? vo | s.oob : vo, s.k0);
+    lds_u8* to = lds + dst + (is_a ? 0 : Cfg::kAStage) + (4 * q + wave) * 1024;
+    if (kNt && !is_a)
+      dma16_nt(s.b, to, kEdge ? vo | s.oob : vo, s.k0);
+    else
+      dma16(is_a ? s.a : s.b, to, kEdge ? vo | s.oob : vo, s.k0);
   };
 
   // ---- fragment reads: rows 16 f + l % 16 of the wave's part.  Lane group
@@ -469,7 +478,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
       else wait_vmcnt<(S - 2) * kD>();
       barrier();
       if constexpr (kExt)
-        if (first && h == 0) scale_dma(t);
+        if (first && h == 0) scale_dma(kSplit ? t % tiles : t);
       const int rst = next_stage(st);
       step(h, st, rst, k + h + S, !(warm && h == 0), edge);
       st = rst;
@@ -515,25 +524,25 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
     // ---- epilogue ---------------------------------------------------------
     bool write_c = !kSplit;
     if constexpr (kSplit) {
-      // The unit's fp32 partial: wave w's 16 blocks at ((t * 4 + w) * 16 +
-      // 4 i + j) KiB of g.split.partial, lane l's 16 bytes at + 16 l (unit
+      // The unit's fp32 partial: wave w's FA x FB blocks at ((t * 4 + w) * FA *
+      // FB + FB i + j) KiB of g.split.partial, lane l's 16 bytes at + 16 l (unit
       // t = slice * tiles + tile).
       constexpr int kCoherent = 16;  // cache policy: sc1
       const int slices = g.split.slices;
       const __amdgpu_buffer_rsrc_t rp = make_rsrc(
-          g.split.partial, (uint32_t)tiles * (uint32_t)slices * 65536u);
+          g.split.partial, (uint32_t)tiles * (uint32_t)slices * (uint32_t)Cfg::kPartial);
       const uint32_t lo = (uint32_t)lane * 16u;
       // Wave-uniform offsets in scalar registers (t's division ran on the
       // VALU): a buffer instruction whose scalar operand sits in a VGPR is
       // wrapped in a readfirstlane loop.
       const uint32_t own_off =
-          (uint32_t)__builtin_amdgcn_readfirstlane((t * 4 + wave) * 16384);
+          (uint32_t)__builtin_amdgcn_readfirstlane((t * 4 + wave) * (Cfg::kPartial / 4));
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < FA; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < FB; ++j)
           store_b128<kCoherent>(__builtin_bit_cast(i32x4, acc[i][j]), rp,
-                                lo + (uint32_t)((4 * i + j) * 1024), own_off);
+                                lo + (uint32_t)((FB * i + j) * 1024), own_off);
       if (g.split.arrivals) {
         const int tile = __builtin_amdgcn_readfirstlane(t % tiles);
         const int own = __builtin_amdgcn_readfirstlane(t / tiles);
@@ -551,42 +560,42 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
           // in flight at a time; the own slice comes from the accumulators,
           // slices past the last read zero (offset out of range: +0, which
           // leaves every sum unchanged).
-          f32x4 sum[4][4];
+          f32x4 sum[FA][FB];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < FA; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) sum[i][j] = f32x4{};
+            for (int j = 0; j < FB; ++j) sum[i][j] = f32x4{};
           for (int q0 = 0; q0 < slices; q0 += 2) {
-            f32x4 v[2][4][4];
+            f32x4 v[2][FA][FB];
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
               const int q = q0 + b;
               const uint32_t so =
-                  (uint32_t)(((q < slices ? q : 0) * tiles + tile) * 4 + wave) * 16384u;
+                  (uint32_t)(((q < slices ? q : 0) * tiles + tile) * 4 + wave) * (uint32_t)(Cfg::kPartial / 4);
               const uint32_t oob = q < slices && q != own ? 0u : kOobOffset;
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
+              for (int i = 0; i < FA; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < FB; ++j)
                   v[b][i][j] = __builtin_bit_cast(
                       f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                 rp, (lo + (uint32_t)((4 * i + j) * 1024)) | oob, so,
+                                 rp, (lo + (uint32_t)((FB * i + j) * 1024)) | oob, so,
                                  kCoherent));
             }
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
               const bool is_own = q0 + b == own;
 #pragma unroll
-              for (int i = 0; i < 4; ++i)
+              for (int i = 0; i < FA; ++i)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < FB; ++j)
                   sum[i][j] += is_own ? acc[i][j] : v[b][i][j];
             }
           }
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
+          for (int i = 0; i < FA; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j];
+            for (int j = 0; j < FB; ++j) acc[i][j] = sum[i][j];
           // Every lane stores the same zero: no branch on the lane.
           __hip_atomic_store(ctr, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           write_c = true;
@@ -679,7 +688,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
                      pack(acc[i][j], i, j));
         compiler_fence();
 #pragma unroll
-        for (int q = 0; q < Cfg::kStoreStage / 1024; ++q) {
+        for (int q = 0; q < Cfg::kRows16 / 1024; ++q) {
           const int x = 64 * q + elane, r = x / kUnits, c = x % kUnits;
           i32x4 v = lds_read16(stg + r * kRow + (((2 * c) ^ (r & kX)) >> 1) * 16);
           if (r & 1) v = i32x4{v[2], v[3], v[0], v[1]};

@@ -1,11 +1,13 @@
-"""AUTO's tiles between 128 x 128 and 256 x 256 (hipgemm_auto_tile): where
-AUTO takes them, and their results against the oracle, bit for bit on ternary
+"""AUTO's tiles other than its schedules' own (hipgemm_auto_tile): where AUTO
+takes them, and their results against the oracle, bit for bit on ternary
 operands (every partial sum exact, in any order).
 
 Shapes end inside a tile in both directions, inside a K-step, or exactly on
 them, run one and several tiles per workgroup, and take 16-byte stores of C or
 not; every output type and epilogue option of the general entry point runs on
-every tile, with canaries around C.
+every tile, with canaries around C.  64-column tiles split K where the call
+brings a workspace: every call runs without one, and twice with one, whose
+counters have to end at zero.
 """
 import numpy as np
 import pytest
@@ -21,8 +23,16 @@ NP = {4: np.uint32, 2: np.uint16, 1: np.uint8}
 
 # shape -> AUTO's tile on 256 CUs
 SHAPES = {
-    (144, 256, 2272): (128, 128),    # K-split plan, run unsplit
-    (190, 237, 2192): (128, 128),    # odd N: 2-byte stores
+    (64, 8192, 8192): (64, 64),      # 2 K-slices
+    (33, 200, 4096): (64, 64),       # 8 K-slices
+    (127, 1001, 4112): (64, 64),     # odd N; K ends inside a step
+    (128, 8192, 8192): (128, 64),    # 2 K-slices
+    (65, 9000, 1040): (128, 64),
+    (144, 256, 2272): (64, 64),      # ragged rows of tiles, K-slices
+    (300, 1000, 4112): (64, 64),
+    (200, 6144, 640): (128, 64),
+    (700, 1501, 528): (128, 64),     # odd N: 2-byte stores
+    (1163, 206, 2112): (128, 128),   # K-split plan, run unsplit
     (4221, 1832, 16): (128, 128),    # two rounds, one K-step
     (2055, 3640, 336): (128, 256),
     (1201, 5891, 240): (128, 256),   # odd N
@@ -45,16 +55,27 @@ def test_auto_tile(shape):
 
 
 def test_auto_tile_keeps_other_choices():
-    """None up to 128 rows, where 256 x 256 tiles fill whole rounds, for the
+    """None up to 32 rows, where 256 x 256 tiles fill whole rounds, for the
     documented column split, or without work."""
-    for M, N, K in [(128, 8192, 8192), (64, 4096, 4096), (8192, 8192, 8192),
+    for M, N, K in [(32, 8192, 8192), (16, 4096, 4096), (8192, 8192, 8192),
                     (4096, 4096, 4096), (8192, 28672, 8192), (4000, 5000, 3584),
-                    (256, 8192, 8192), (512, 512, 512), (300, 300, 0), (0, 64, 64)]:
+                    (300, 300, 0), (0, 64, 64)]:
         assert hg.auto_tile(M, N, K) is None, (M, N, K)
 
 
+def test_short_workspace_is_refused():
+    """Whichever tile runs, AUTO refuses a workspace below
+    hipgemm_workspace_size (before any launch)."""
+    fake = 1 << 20
+    for M, N, K in SHAPES:
+        need = hg.workspace_size(M, N, K, 0)
+        if need:
+            assert hg.gemm_raw_ws(fake, fake, fake, M, N, K, K, K, N, 0, 0, 0, fake,
+                                  need - 256) == hg.hipErrorInvalidValue
+
+
 def run(torch, A, B, out, ldc, *, fb=0, act=0, sa=None, sr=None, sc=None, bias=None,
-        so=None):
+        so=None, ws=None):
     M, K = A.shape
     N = B.shape[0]
     es = ES[out]
@@ -68,7 +89,9 @@ def run(torch, A, B, out, ldc, *, fb=0, act=0, sa=None, sr=None, sc=None, bias=N
                     M=M, N=N, K=K, lda=K, ldb=K, ldc=ldc, b_format=fb,
                     out_dtype=out, activation=act, scale_a=ptr["sa"],
                     scale_rows=ptr["sr"], scale_cols=ptr["sc"], bias=ptr["bias"],
-                    scale_out=ptr["so"])
+                    scale_out=ptr["so"],
+                    workspace=0 if ws is None else ws.data_ptr(),
+                    workspace_bytes=0 if ws is None else ws.numel())
     assert hg.gemm_desc_raw(d, torch.cuda.current_stream().cuda_stream) == 0
     torch.cuda.synchronize()
     got = buf.cpu().numpy().reshape(M + 4, ldc * es)
@@ -76,6 +99,18 @@ def run(torch, A, B, out, ldc, *, fb=0, act=0, sa=None, sr=None, sc=None, bias=N
              np.all(got[2:M + 2, N * es:] == 0xA5))
     C = np.ascontiguousarray(got[2:M + 2, :N * es]).view(NP[es])
     return C, guard
+
+
+def runs(torch, A, B, out, ldc, want, **kw):
+    """Without a workspace, then twice with one."""
+    M, K = A.shape
+    need = hg.workspace_size(M, B.shape[0], K, 0)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda") if need else None
+    for w in (None, ws, ws) if need else (None,):
+        C, guard = run(torch, A, B, out, ldc, ws=w, **kw)
+        assert guard, "write outside M x N"
+        assert np.array_equal(C, want), f"{int((C != want).sum())} of {C.size} differ"
+        assert w is None or not w[:16384].cpu().numpy().any(), "counters not left zero"
 
 
 @pytest.mark.gpu
@@ -87,10 +122,8 @@ def test_tile_bit_exact(gpu, oracle, shape):
         say(f"case tile {SHAPES[shape]} M={M} N={N} K={K} fb={fb} ldc=N+{pad}")
         A = TERN[0][rng.integers(0, 3, (M, K))]
         B = TERN[fb][rng.integers(0, 3, (N, K))]
-        C, guard = run(gpu, A, B, po.OUT_BF16, N + pad, fb=fb, sa=[0.5])
         want = oracle.gemm_ex(A, B, b_fmt=fb, scale_a=0.5)
-        assert guard, "write outside M x N"
-        assert np.array_equal(C, want), f"{int((C != want).sum())} of {C.size} differ"
+        runs(gpu, A, B, po.OUT_BF16, N + pad, want, fb=fb, sa=[0.5])
 
 
 @pytest.mark.gpu
@@ -108,10 +141,8 @@ def test_tile_epilogue(gpu, oracle, shape, out):
     so = 0.25 if out == po.OUT_FP8 else None
     for act in (po.ACT_NONE, po.ACT_RELU):
         say(f"case tile {SHAPES[shape]} M={M} N={N} K={K} out={out} act={act}")
-        C, guard = run(gpu, A, B, out, N + 8, fb=1, act=act, sa=[0.5], sr=sr, sc=sc,
-                       bias=bias, so=None if so is None else [so])
         want = oracle.gemm_ex(A, B, b_fmt=1, out=out, act=act, scale_a=0.5,
                               scale_rows=sr, scale_cols=sc, bias=bias,
                               scale_out=so or 1.0)
-        assert guard, "write outside M x N"
-        assert np.array_equal(C, want), f"{int((C != want).sum())} of {C.size} differ"
+        runs(gpu, A, B, out, N + 8, want, fb=1, act=act, sa=[0.5], sr=sr, sc=sc,
+             bias=bias, so=None if so is None else [so])
