@@ -21,6 +21,7 @@ the reference has no error path (fp8_4wave.hpp has no shape checks).
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 import re
 from typing import Optional
@@ -84,6 +85,12 @@ class GemmDesc(ctypes.Structure):
             setattr(self, k, v or (None if k in _PTR_FIELDS else 0))
 
 
+class _Desc(ctypes.Structure):
+    """hipgemm_gemm_desc again, built from positional values: a call of gemm()
+    spent 7 us in GemmDesc's keyword loop, 1.5 here."""
+    _fields_ = GemmDesc._fields_
+
+
 _PTR_FIELDS = {"A", "B_T", "C", "scale_a", "scale_b", "scale_rows",
                "scale_cols", "bias", "workspace", "mx_scale_a", "mx_scale_b",
                "scale_out"}
@@ -129,7 +136,7 @@ def lib() -> ctypes.CDLL:
                                                ci, vp, vp, ci, vp,
                                                ctypes.c_size_t, vp]
     L.hipgemm_fp8_gemm_bf16_rowcol.restype = ci
-    L.hipgemm_gemm.argtypes = [ctypes.POINTER(GemmDesc), vp]
+    L.hipgemm_gemm.argtypes = [vp, vp]  # a hipgemm_gemm_desc by reference
     L.hipgemm_gemm.restype = ci
     L.hipgemm_gemm_noalloc.argtypes = [ctypes.POINTER(GemmDesc), vp]
     L.hipgemm_gemm_noalloc.restype = ci
@@ -217,7 +224,7 @@ def gemm_raw_rowcol(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int,
 
 def gemm_desc_raw(desc: "GemmDesc", stream: int = 0) -> int:
     """Call hipgemm_gemm; returns hipError_t."""
-    return int(lib().hipgemm_gemm(ctypes.byref(desc), stream or None))
+    return int(lib().hipgemm_gemm(ctypes.addressof(desc), stream or None))
 
 
 def gemm_desc_noalloc_raw(desc: "GemmDesc", stream: int = 0) -> int:
@@ -318,6 +325,7 @@ def lds_stage_slot(row: int, piece: int) -> int:
 # -- torch convenience layer ----------------------------------------------
 
 
+@functools.lru_cache(maxsize=1)
 def _torch():
     import torch  # noqa: WPS433 - torch is optional for the raw ABI
     return torch
@@ -374,9 +382,24 @@ def _mx_ptr(t, rows, K, name):
     return t.data_ptr()
 
 
-def _gemm_operands(a, b_t, out, variant, stream, out_dtype=None):
+# Workspace bytes by sizes and options (a pure function of them on one GPU
+# model; the C call and a descriptor cost 2 us per GEMM).
+@functools.lru_cache(maxsize=4096)
+def _ws_bytes(device: int, M: int, N: int, K: int, variant: int,
+              a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
+              mx: bool = False) -> int:
+    if M <= 0 or N <= 0:
+        return 0
+    if not mx and a_format <= FMT_E5M2 and b_format <= FMT_E5M2:
+        return workspace_size(M, N, K, variant)
+    d = GemmDesc(M=M, N=N, K=K, a_format=a_format, b_format=b_format,
+                 variant=variant, mx_scale_a=int(mx), mx_scale_b=int(mx))
+    return int(lib().hipgemm_gemm_workspace_size(ctypes.byref(d)))
+
+
+def _gemm_operands(a, b_t, out, stream, out_dtype=None):
     """Shared argument handling of the torch entry points: shapes, strides,
-    output (out_dtype, default bfloat16), stream and workspace."""
+    output (out_dtype, default bfloat16) and the stream's handle."""
     torch = _torch()
     out_dtype = out_dtype or torch.bfloat16
     a = _as_bytes_2d(a, "a")
@@ -392,17 +415,12 @@ def _gemm_operands(a, b_t, out, variant, stream, out_dtype=None):
           (M > 0 and N > 0 and out.stride(1) != 1)):
         raise HipGemmError(f"out must be a (M, N) {out_dtype} tensor with unit "
                            "column stride", hipErrorInvalidValue)
-    if stream is None:
-        stream = torch.cuda.current_stream(a.device)
+    handle = (torch._C._cuda_getCurrentRawStream(a.get_device())
+              if stream is None else stream.cuda_stream)
     lda = a.stride(0) if (M > 1 and K > 0) else max(K, 16)
     ldb = b_t.stride(0) if (N > 1 and K > 0) else max(K, 16)
     ldc = out.stride(0) if M > 1 else max(N, 1)
-    nbytes = workspace_size(M, N, K, variant) if M > 0 and N > 0 else 0
-    ws = _workspace(a.device, stream, nbytes) if nbytes else None
-    if ws is None:
-        nbytes = 0
-    return (a, b_t, out, M, N, K, lda, ldb, ldc,
-            ws.data_ptr() if ws is not None else 0, nbytes, stream)
+    return a, b_t, out, M, N, K, lda, ldb, ldc, handle
 
 
 def fp8_gemm_bf16(a, b_t, scale_a=None, scale_b=None, out=None,
@@ -415,21 +433,21 @@ def fp8_gemm_bf16(a, b_t, scale_a=None, scale_b=None, out=None,
     stride; allocated if None.  Runs on `stream` (a torch.cuda.Stream) or the
     current stream.
     """
-    a, b_t, out, M, N, K, lda, ldb, ldc, ws, nbytes, stream = _gemm_operands(
-        a, b_t, out, variant, stream)
+    a, b_t, out, M, N, K, lda, ldb, ldc, handle = _gemm_operands(a, b_t, out, stream)
+    ws, nbytes = _stream_workspace(a, stream, handle,
+                                   _ws_bytes(a.get_device(), M, N, K, variant))
+    sa, sb = _scale_ptr(scale_a, "scale_a"), _scale_ptr(scale_b, "scale_b")
     if not ws:
         # No workspace (none needed, or the stream is being captured): the
         # entry point that takes none.
-        code = gemm_raw(a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
-                        lda, ldb, ldc, _scale_ptr(scale_a, "scale_a"),
-                        _scale_ptr(scale_b, "scale_b"), variant,
-                        stream.cuda_stream)
+        code = lib().hipgemm_fp8_gemm_bf16(
+            a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K, lda, ldb, ldc,
+            sa, sb, variant, handle)
         _check(code, "hipgemm_fp8_gemm_bf16")
         return out
-    code = gemm_raw_ws(a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
-                       lda, ldb, ldc, _scale_ptr(scale_a, "scale_a"),
-                       _scale_ptr(scale_b, "scale_b"), variant, ws, nbytes,
-                       stream.cuda_stream)
+    code = lib().hipgemm_fp8_gemm_bf16_ws(
+        a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K, lda, ldb, ldc, sa,
+        sb, variant, ws, nbytes, handle)
     _check(code, "hipgemm_fp8_gemm_bf16_ws")
     return out
 
@@ -454,8 +472,7 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     mx_scale_a / mx_scale_b: MX block scales packed by mx_pack_scales
     (both or neither)."""
     torch = _torch()
-    fmts = {torch.float8_e4m3fn: FMT_E4M3, torch.float8_e5m2: FMT_E5M2,
-            torch.float4_e2m1fn_x2: FMT_FP4_E2M1}
+    fmts, codes = _dtype_codes()
     a_format = fmts.get(a.dtype, a_format)
     b_format = fmts.get(b_t.dtype, b_format)
     if a.dtype == torch.float4_e2m1fn_x2:
@@ -463,8 +480,6 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     if b_t.dtype == torch.float4_e2m1fn_x2:
         b_t = b_t.view(torch.uint8)
     out_dtype = out_dtype or (out.dtype if out is not None else torch.bfloat16)
-    codes = {torch.bfloat16: OUT_BF16, torch.float16: OUT_F16,
-             torch.float32: OUT_F32, torch.float8_e4m3fn: OUT_FP8_E4M3}
     if out_dtype not in codes:
         raise HipGemmError("out_dtype must be bfloat16, float16, float32 or "
                            "float8_e4m3fn", hipErrorInvalidValue)
@@ -473,10 +488,10 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
                            hipErrorInvalidValue)
     if out is not None and out.dtype != out_dtype:
         raise HipGemmError("out has the wrong dtype", hipErrorInvalidValue)
-    a, b_t, out, M, N, K, lda, ldb, ldc, ws, nbytes, stream = _gemm_operands(
+    a, b_t, out, M, N, K, lda, ldb, ldc, handle = _gemm_operands(
         a.view(torch.uint8) if a.dtype == torch.float8_e5m2 else a,
         b_t.view(torch.uint8) if b_t.dtype == torch.float8_e5m2 else b_t,
-        out, variant, stream, out_dtype)
+        out, stream, out_dtype)
     if a_format == FMT_FP4_E2M1 or b_format == FMT_FP4_E2M1:
         K *= 2  # elements: two per byte
     elif a_format in (FMT_FP6_E2M3, FMT_FP6_E3M2):
@@ -485,27 +500,33 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
                                "row length in bytes must be a multiple of 3",
                                hipErrorInvalidValue)
         K = K // 3 * 4  # elements: four per three bytes
-    d = GemmDesc(A=a.data_ptr(), B_T=b_t.data_ptr(), C=out.data_ptr(), M=M,
-                 N=N, K=K, lda=lda, ldb=ldb, ldc=ldc, a_format=a_format,
-                 b_format=b_format,
-                 out_dtype=codes[out_dtype],
-                 activation=ACTIVATIONS[activation],
-                 scale_a=_scale_ptr(scale_a, "scale_a"),
-                 scale_b=_scale_ptr(scale_b, "scale_b"),
-                 scale_rows=_vector_ptr(scale_rows, M, "scale_rows"),
-                 scale_cols=_vector_ptr(scale_cols, N, "scale_cols"),
-                 bias=_vector_ptr(bias, N, "bias"), variant=variant,
-                 workspace=ws, workspace_bytes=nbytes,
-                 mx_scale_a=_mx_ptr(mx_scale_a, M, K, "mx_scale_a"),
-                 mx_scale_b=_mx_ptr(mx_scale_b, N, K, "mx_scale_b"),
-                 scale_out=_scale_ptr(scale_out, "scale_out"))
-    need = int(lib().hipgemm_gemm_workspace_size(ctypes.byref(d)))
-    if need != nbytes:  # the formats and MX scales decide the schedule
-        w = _workspace(a.device, stream, need) if need else None
-        d.workspace = w.data_ptr() if w is not None else None
-        d.workspace_bytes = need if w is not None else 0
-    _check(gemm_desc_raw(d, stream.cuda_stream), "hipgemm_gemm")
+    mx_a = _mx_ptr(mx_scale_a, M, K, "mx_scale_a")
+    mx_b = _mx_ptr(mx_scale_b, N, K, "mx_scale_b")
+    ptrs = (_scale_ptr(scale_a, "scale_a"), _scale_ptr(scale_b, "scale_b"),
+            _vector_ptr(scale_rows, M, "scale_rows"),
+            _vector_ptr(scale_cols, N, "scale_cols"), _vector_ptr(bias, N, "bias"))
+    so = _scale_ptr(scale_out, "scale_out")
+    ws, nbytes = _stream_workspace(
+        a, stream, handle, _ws_bytes(a.get_device(), M, N, K, variant, a_format,
+                                     b_format, bool(mx_a or mx_b)))
+    d = _Desc(_DESC_BYTES, a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
+              lda, ldb, ldc, a_format, b_format, codes[out_dtype],
+              ACTIVATIONS[activation], *ptrs, variant, ws, nbytes, mx_a, mx_b, so)
+    _check(lib().hipgemm_gemm(ctypes.addressof(d), handle), "hipgemm_gemm")
     return out
+
+
+_DESC_BYTES = ctypes.sizeof(_Desc)
+
+
+@functools.lru_cache(maxsize=1)
+def _dtype_codes():
+    """Operand formats and output codes by torch dtype."""
+    torch = _torch()
+    return ({torch.float8_e4m3fn: FMT_E4M3, torch.float8_e5m2: FMT_E5M2,
+             torch.float4_e2m1fn_x2: FMT_FP4_E2M1},
+            {torch.bfloat16: OUT_BF16, torch.float16: OUT_F16,
+             torch.float32: OUT_F32, torch.float8_e4m3fn: OUT_FP8_E4M3})
 
 
 def fp8_gemm_bf16_rowcol(a, b_t, scale_rows=None, scale_cols=None, out=None,
@@ -517,13 +538,14 @@ def fp8_gemm_bf16_rowcol(a, b_t, scale_rows=None, scale_cols=None, out=None,
     elements); either may be None for all ones.  variant 1 (the 32x32x64
     schedule) is not available here.
     """
-    a, b_t, out, M, N, K, lda, ldb, ldc, ws, nbytes, stream = _gemm_operands(
-        a, b_t, out, variant, stream)
+    a, b_t, out, M, N, K, lda, ldb, ldc, handle = _gemm_operands(a, b_t, out, stream)
+    ws, nbytes = _stream_workspace(a, stream, handle,
+                                   _ws_bytes(a.get_device(), M, N, K, variant))
     code = gemm_raw_rowcol(a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N,
                            K, lda, ldb, ldc,
                            _vector_ptr(scale_rows, M, "scale_rows"),
                            _vector_ptr(scale_cols, N, "scale_cols"), variant,
-                           ws, nbytes, stream.cuda_stream)
+                           ws, nbytes, handle)
     _check(code, "hipgemm_fp8_gemm_bf16_rowcol")
     return out
 
@@ -540,6 +562,22 @@ def fp8_gemm_bf16_rowcol(a, b_t, scale_rows=None, scale_cols=None, out=None,
 # split K unsplit (include/hipgemm.h).
 _workspaces: dict = {}
 _retired: list = []
+
+
+def _stream_workspace(a, stream, handle: int, nbytes: int):
+    """(pointer, nbytes) of the workspace of a's device and `stream` (None: the
+    current one; `handle` is its handle), or (0, 0) where none is needed or
+    none may be allocated."""
+    if not nbytes:
+        return 0, 0
+    ws = _workspaces.get((a.get_device(), handle))
+    if ws is None or ws.numel() < nbytes:
+        if stream is None:
+            stream = _torch().cuda.current_stream(a.device)
+        ws = _workspace(a.device, stream, nbytes)
+        if ws is None:
+            return 0, 0
+    return ws.data_ptr(), nbytes
 
 
 def _workspace(device, stream, nbytes: int):
