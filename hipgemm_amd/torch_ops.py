@@ -165,18 +165,23 @@ def quantize_rows(x: torch.Tensor):
     (hipgemm_quantize_rows_e4m3), with the same results bit for bit; under
     autograd, a transform or a trace, on the CPU and for other layouts these
     are tensor operations."""
-    if (_plain_eager(x) and x.dim() == 2 and x.dtype in _QUANT_TYPES
-            and x.numel() > 0 and x.stride(1) == 1
-            and x.stride(0) >= x.shape[1]
-            and x.shape[0] < 2 ** 31 and x.shape[1] < 2 ** 31):
-        M, K = x.shape
-        q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=x.device)
-        s = torch.empty((M,), dtype=torch.float32, device=x.device)
-        _check(int(lib().hipgemm_quantize_rows_e4m3(
-            x.data_ptr(), _QUANT_TYPES[x.dtype], M, K, x.stride(0), q.data_ptr(),
-            s.data_ptr(), torch.cuda.current_stream(x.device).cuda_stream or None)),
-            "hipgemm_quantize_rows_e4m3")
-        return q, s
+    return _quantize_rows(x, _plain_eager(x))
+
+
+def _quantize_rows(x: torch.Tensor, plain: bool):
+    """quantize_rows, with _plain_eager(x) known."""
+    kind = _QUANT_TYPES.get(x.dtype)
+    if plain and kind is not None and x.dim() == 2:
+        (M, K), (ld, unit) = x.shape, x.stride()
+        if 0 < M < 2 ** 31 and 0 < K < 2 ** 31 and unit == 1 and ld >= K:
+            dev = x.device
+            q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=dev)
+            s = torch.empty(M, dtype=torch.float32, device=dev)
+            _check(lib().hipgemm_quantize_rows_e4m3(
+                x.data_ptr(), kind, M, K, ld, q.data_ptr(), s.data_ptr(),
+                torch._C._cuda_getCurrentRawStream(dev.index)),
+                "hipgemm_quantize_rows_e4m3")
+            return q, s
     return _quantize_rows_ops(x)
 
 
@@ -237,19 +242,20 @@ class Fp8Linear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         lead = x.shape[:-1]
         x2 = x.reshape(-1, self.in_features)
-        q, s = quantize_rows(x2)
+        plain = _plain_eager(x2)
+        q, s = _quantize_rows(x2, plain)
         # Where nothing watches the operations (as for quantize_rows), the
         # call itself instead of the operator around it: the dispatcher and the
         # operator's wrappers take about 20 us of host time.
-        gemm = (_gemm if _plain_eager(x2) and self._plain_buffers() else
-                torch.ops.hipgemm.gemm)
-        y = gemm(q, self.weight, scale_rows=s, scale_cols=self.weight_scale,
-                 bias=self.bias, activation=self.activation,
-                 variant=self.variant)
-        return y.reshape(*lead, self.out_features)
+        w, sw, bias = self.weight, self.weight_scale, self.bias
+        gemm = _gemm if plain and _plain_buffers(w, sw, bias) else torch.ops.hipgemm.gemm
+        y = gemm(q, w, scale_rows=s, scale_cols=sw, bias=bias,
+                 activation=self.activation, variant=self.variant)
+        return y if x.dim() == 2 else y.reshape(*lead, self.out_features)
 
-    def _plain_buffers(self) -> bool:
-        grad = torch.is_grad_enabled()
-        return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter)
-                                 and not (grad and t.requires_grad))
-                   for t in (self.weight, self.weight_scale, self.bias))
+
+def _plain_buffers(*tensors) -> bool:
+    grad = torch.is_grad_enabled()
+    return all(t is None or (type(t) in (torch.Tensor, torch.nn.Parameter)
+                             and not (grad and t.requires_grad))
+               for t in tensors)

@@ -138,3 +138,25 @@ def test_watched_calls_keep_the_tensor_operations(gpu, monkeypatch):
     with gpu.no_grad():
         monkeypatch.undo()
         same(ops.quantize_rows(r))
+
+
+@pytest.mark.gpu
+def test_layer_equals_operator_path(gpu, monkeypatch):
+    """Fp8Linear's direct call against the operator it takes when something
+    watches the operations: the same bits, for 2-D, 3-D and empty inputs."""
+    gpu.manual_seed(9)
+    layer = ops.Fp8Linear.from_linear(gpu.nn.Linear(256, 384).cuda(), activation="silu")
+    for shape in ((40, 256), (2, 3, 256), (0, 256), (1, 256)):
+        say(f"case fp8-linear direct x={shape}")
+        x = gpu.randn(shape, device="cuda", dtype=gpu.bfloat16)
+        got = layer(x)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "_plain_eager", lambda t: False)
+            want = layer(x)
+        gpu.cuda.synchronize()
+        assert got.shape == want.shape == (*shape[:-1], 384)
+        assert gpu.equal(got.view(gpu.int16), want.view(gpu.int16))
+    x = gpu.randn(4, 256, device="cuda", requires_grad=True)
+    assert layer(x).requires_grad
+    with gpu.no_grad():
+        assert not layer(x).requires_grad
