@@ -27,20 +27,51 @@ __global__ __launch_bounds__(256, 1) void k_fp8_gemm_t128_split_mx(GemmArgs g) {
   gemm_t128_body<true, false, kFmt, kActNone, kOutBf16, true, true>(g, (lds_u8*)lds);
 }
 
-// One thread per packed byte (layout of MxArgs): byte f of step st of lane l
-// in (W, p) is the scale of row 128 W + 16 f + l % 16, K-block
-// 4 (2 p + st) + l / 16; 127 (1.0) past the rows or blocks of the source.
+// The packed layout (MxArgs): byte f of step st of lane l in (W, p) is the
+// scale of row 128 W + 16 f + l % 16, K-block 4 (2 p + st) + l / 16; 127 (1.0)
+// past the rows or blocks of the source.
+// One wave per 1 KiB of the packed layout (128 rows W, step pair p): a lane
+// loads the 8 scales of rows `lane` and lane + 64, scatters their bytes through
+// the wave's 1 KiB of LDS and stores 16 bytes.  One thread per packed
+// byte did two divisions for one scattered byte load: in a graph, 4096 x 8192
+// 4.9 -> 3.1 us, 8192 x 8192 7.5 -> 3.5, 128 x 4096 3.0 -> 2.4.  kWide: the source's rows start on 8 bytes, the packed buffer on 16;
+// else byte by byte.
+template <bool kWide>
 __global__ __launch_bounds__(256) void k_mx_pack(const uint8_t* src, int rows,
                                                  int kblocks, int ld, int pairs,
-                                                 uint8_t* dst, size_t n) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const int f = (int)(i & 7), st = (int)((i >> 3) & 1), l = (int)((i >> 4) & 63);
-  const size_t wp = i >> 10;
-  const int p = (int)(wp % pairs), W = (int)(wp / pairs);
-  const int row = 128 * W + 16 * f + (l & 15);
-  const int blk = 4 * (2 * p + st) + (l >> 4);
-  dst[i] = (row < rows && blk < kblocks) ? src[(size_t)row * ld + blk] : 127;
+                                                 uint8_t* dst, int chunks) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[4 * 1024];
+  const int lane = lane_id(), wave = wave_id();
+  const int chunk = blockIdx.x * 4 + wave;
+  if (chunk >= chunks) return;
+  const int W = chunk / pairs, p = chunk % pairs;
+  uint8_t* mine = lds + wave * 1024;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = 64 * h + lane, row = 128 * W + r, f = r >> 4;
+    const int left = row < rows ? kblocks - 8 * p : 0;  // scales of the row here
+    const uint8_t* s = src + (size_t)row * ld + 8 * p;
+    uint64_t v = 0x7f7f7f7f7f7f7f7full;  // padding: 1.0
+    if (kWide && left >= 8) {
+      v = *reinterpret_cast<const uint64_t*>(s);
+    } else {
+      for (int b = 0; b < left && b < 8; ++b)
+        v = (v & ~(0xffull << (8 * b))) | ((uint64_t)s[b] << (8 * b));
+    }
+    // Block b of the pair: step b / 4, lane group b % 4.
+#pragma unroll
+    for (int b = 0; b < 8; ++b)
+      mine[((b & 3) * 16 + (r & 15)) * 16 + (b >> 2) * 8 + f] = (uint8_t)(v >> (8 * b));
+  }
+  // The wave's own region: its LDS operations complete in order.
+  compiler_fence();
+  uint8_t* to = dst + (size_t)chunk * 1024 + lane * 16;
+  if constexpr (kWide) {
+    *reinterpret_cast<i32x4*>(to) = lds_read16((lds_u8*)mine + lane * 16);
+  } else {
+#pragma unroll
+    for (int b = 0; b < 16; ++b) to[b] = mine[lane * 16 + b];
+  }
 }
 
 }  // namespace
@@ -74,10 +105,13 @@ hipError_t mx_pack(const uint8_t* src, int rows, int K, int ld, uint8_t* dst,
                    hipStream_t stream) {
   const size_t n = mx_packed_bytes(rows, K);
   if (n == 0) return hipSuccess;
-  int kblocks = (K + 31) / 32, pairs = mx_pairs(K);
-  void* args[] = {&src, &rows, &kblocks, &ld, &pairs, &dst, const_cast<size_t*>(&n)};
-  return hipLaunchKernel((const void*)&k_mx_pack, dim3((unsigned)((n + 255) / 256)),
-                         dim3(256), args, 0, stream);
+  int kblocks = (K + 31) / 32, pairs = mx_pairs(K), chunks = (int)(n / 1024);
+  const bool wide = ld % 8 == 0 && reinterpret_cast<uintptr_t>(src) % 8 == 0 &&
+                    reinterpret_cast<uintptr_t>(dst) % 16 == 0;
+  const void* fn = wide ? (const void*)&k_mx_pack<true> : (const void*)&k_mx_pack<false>;
+  void* args[] = {&src, &rows, &kblocks, &ld, &pairs, &dst, &chunks};
+  return hipLaunchKernel(fn, dim3((unsigned)((chunks + 3) / 4)), dim3(256), args, 0,
+                         stream);
 }
 
 }  // namespace kernels
