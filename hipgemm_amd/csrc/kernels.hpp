@@ -70,10 +70,10 @@ const void* narrow_ext_wide(int tile, int mode, const Key& k);    // knarrow_ext
 // `stream` unless the stream is being captured.  nullptr with *err set on
 // failure.
 void* noalloc_scratch(hipStream_t stream, hipError_t* err);
-// Packs [rows][ceil(K/32)] E8M0 scales (row stride ld) into MxArgs' layout.
 // Per-row e4m3 quantisation (kquant.hip); type: HIPGEMM_IN_*.
 hipError_t quantize_rows(const void* x, int type, int M, int K, long long ldx,
                          void* q, float* s, hipStream_t stream);
+// Packs [rows][ceil(K/32)] E8M0 scales (row stride ld) into MxArgs' layout.
 hipError_t mx_pack(const uint8_t* src, int rows, int K, int ld, uint8_t* dst,
                    hipStream_t stream);
 
