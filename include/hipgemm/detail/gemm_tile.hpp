@@ -40,14 +40,14 @@
 // the others (the step K ends inside, padding, the next tile's steps) go
 // through a per-lane select, in a copy of the step of their own.
 //
-// K order: where a unit's K range is whole steps, the workgroups of XCD x
-// (blockIdx % 8) start it at step x * steps / 8 and wrap around (not with MX
-// scales, whose scale words follow the plain order).  Started together at
-// step 0, every workgroup's DMA of a step falls at the same offset of each
-// operand row, and with row strides that are a multiple of 4096 bytes all
-// those rows meet at one offset within 4 KiB -- which measured as an
-// HBM-bound stall; one start per XCD keeps the workgroups of an XCD (which
-// share operand panels in their L2) in step.  Same process, 128 x 128 tiles,
+// K order: the workgroups of XCD x (blockIdx % 8) start a unit's whole steps
+// at step x * whole / 8 of them and wrap around; a step that the unit's K range
+// ends inside comes last (no start but 0 with MX scales, whose scale words
+// follow the plain order).  Started together at step 0, every workgroup's DMA
+// of a step falls at the same offset of each operand row, and with row strides
+// that are a multiple of 4096 bytes all those rows meet at one offset within
+// 4 KiB -- which measured as an HBM-bound stall; one start per XCD keeps the
+// workgroups of an XCD (which share operand panels in their L2) in step.  Same process, 128 x 128 tiles,
 // against starting at step 0: 40 x 28672 x 4096 +19 %, 16 x 28672 x 4096
 // +24 %, 64 x 16384 x 8192 +29 %, 4096 x 1536 x 4096 +5 %, 512 x 4096 x 8192
 // and 2048 x 2048 x 8192 within 1 %.  The fp32 sums run in that rotated order
@@ -188,7 +188,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
 
   // Buffer resources of a unit's A rows and B_T rows (rows past M / N read
   // zero; none past the walk's end), its K range [k0, kend), the whole steps
-  // it starts with, and the step it starts at (K order, above).
+  // of it, and the one it starts at (K order, above).
   struct Src {
     __amdgpu_buffer_rsrc_t a, b;
     int k0, kend, full, rot;
@@ -205,9 +205,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
     const int k0 = __builtin_amdgcn_readfirstlane(slice * steps * kStepBytes);
     const int kend = min(K, k0 + steps * kStepBytes);
     const int full = max(0, kend - k0) / kStepBytes;
-    const int rot = !kMx && full == steps
-                        ? (int)((blockIdx.x & 7u) * (unsigned)steps / 8u)
-                        : 0;
+    const int rot = kMx ? 0 : (int)((blockIdx.x & 7u) * (unsigned)full / 8u);
     return Src{make_rsrc(g.A + (size_t)c.m * Cfg::kBM * g.lda,
                          (uint32_t)ra * (uint32_t)g.lda),
                make_rsrc(g.B + (size_t)c.n * Cfg::kBN * g.ldb,
@@ -228,9 +226,10 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& g, lds_u8* lds) {
     constexpr bool kEdge = decltype(edge)::value;
     const bool next = kEdge && d >= steps_pad;
     const int dd = next ? d - steps_pad : d;
+    const int full = next ? nxt.full : cur.full;
     int dr = dd + (next ? nxt.rot : cur.rot);
-    if (dr >= steps) dr -= steps;
-    if (kEdge && dd >= steps) dr = dd;  // padding: past the range
+    if (dr >= full) dr -= full;
+    if (kEdge && dd >= full) dr = dd;  // the step K ends inside, padding
     uint32_t k0 = (uint32_t)((next ? nxt.k0 : cur.k0) + dr * kStepBytes);
     asm volatile("" : "+s"(k0));
     uint32_t oob = 0;

@@ -146,3 +146,25 @@ def test_tile_epilogue(gpu, oracle, shape, out):
                               scale_out=so or 1.0)
         runs(gpu, A, B, out, N + 8, want, fb=1, act=act, sa=[0.5], sr=sr, sc=sc,
              bias=bias, so=None if so is None else [so])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tail", [0, 16, 112])
+def test_each_xcd_starts_at_its_own_step(gpu, tail):
+    """Workgroups on different XCDs walk K from different steps, also where K
+    ends inside a step.  Step 0 adds 2^23 and every other one 0.5, which is
+    lost on top of that, so the fp32 sum grows with the steps that came before
+    step 0; every tile (one per workgroup) has the same operands."""
+    torch = gpu
+    M, N, K = 128, 128 * 32, 8 * 128 + tail
+    say(f"case start steps tile128 M={M} N={N} K={K}")
+    A, B = np.full((M, K), 0x38, np.uint8), np.zeros((N, K), np.uint8)
+    A[:, :128] = B[:, :128] = 0x78  # 256 * 256 * 128 = 2^23
+    B[:, 128::128] = 0x30           # 1 * 0.5
+    a, b = to_dev(torch, A), to_dev(torch, B)
+    c = hg.gemm(a, b, out_dtype=torch.float32, variant=hg.VARIANTS["tile128"])
+    tiles = c.cpu().numpy().reshape(M, 32, 128)
+    sums = tiles[0, :, 0]
+    assert np.all(tiles == sums[None, :, None])
+    assert np.all((sums >= 2.0 ** 23) & (sums <= 2.0 ** 23 + 4)), sums
+    assert len(set(sums)) > 1, sums
