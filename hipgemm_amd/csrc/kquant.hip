@@ -25,6 +25,8 @@ using namespace detail;
 
 constexpr int kThreads = 256;
 constexpr int kCache = 8;  // 16-byte loads of a row a thread keeps
+// Rows, and so workgroups, of a launch (one of 2^32 threads is refused).
+constexpr int kMaxRows = 1 << 23;
 
 struct QuantArgs {
   const uint8_t* x;
@@ -208,7 +210,17 @@ hipError_t quantize_rows(const void* x, int type, int M, int K, long long ldx,
     default: return hipErrorInvalidValue;
   }
   void* args[] = {&g};
-  return hipLaunchKernel(fn, dim3((unsigned)M), dim3(kThreads), args, 0, stream);
+  // Launches of at most kMaxRows rows (a multiple of 16, so that q keeps its
+  // alignment from one to the next).
+  for (;;) {
+    const int rows = M < kMaxRows ? M : kMaxRows;
+    const hipError_t e =
+        hipLaunchKernel(fn, dim3((unsigned)rows), dim3(kThreads), args, 0, stream);
+    if (e != hipSuccess || (M -= rows) == 0) return e;
+    g.x += rows * ldx * es;
+    g.q += (long long)rows * K;
+    g.s += rows;
+  }
 }
 
 }  // namespace kernels

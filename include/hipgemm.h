@@ -345,7 +345,7 @@ hipError_t hipgemm_mx_pack_scales(const void *src, int rows, int K, int ld,
  * maximum is 0 or NaN; q[m, k] (M x K packed bytes) = e4m3 of x[m, k] / s[m]
  * clamped to +-448, round to nearest even, NaN kept.  So x ~= q * s[m], and q, s
  * are hipgemm_gemm's A and scale_rows.  x aligned to its type, s to 4 bytes,
- * ldx >= K; M == 0 or K == 0 is a no-op.  One launch on `stream`.
+ * ldx >= K; M == 0 or K == 0 is a no-op.  One launch on `stream` per 2^23 rows.
  * No reference counterpart (the reference takes e4m3 operands as they are).
  */
 enum { HIPGEMM_IN_F32 = 0, HIPGEMM_IN_BF16 = 1, HIPGEMM_IN_F16 = 2 };

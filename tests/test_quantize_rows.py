@@ -60,6 +60,31 @@ def test_kernel_equals_tensor_operations(gpu, dtype, shape):
     check(big[:, 1:shape[1] + 1], "strided, unaligned rows")
 
 
+def entry(torch, x):
+    """q, s of hipgemm_quantize_rows_e4m3 itself."""
+    M, K = x.shape
+    q = torch.full((M, K), 0x55, dtype=torch.uint8, device="cuda")
+    s = torch.full((M,), -1.0, device="cuda")
+    assert hg.lib().hipgemm_quantize_rows_e4m3(
+        x.data_ptr(), ops._QUANT_TYPES[x.dtype], M, K, x.stride(0), q.data_ptr(),
+        s.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    return q, s
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [3, 8])
+def test_more_rows_than_one_launch_has_workgroups(gpu, K):
+    """2^24 rows and a few: a workgroup per row would be a launch of 2^32
+    threads."""
+    M = 2 ** 24 + 3
+    say(f"case quantize M={M} K={K} bf16")
+    g = gpu.Generator(device="cuda").manual_seed(5)
+    x = gpu.randn((M, K), generator=g, device="cuda", dtype=gpu.bfloat16)
+    q, s = entry(gpu, x)
+    rq, rs = ops._quantize_rows_ops(x)
+    assert gpu.equal(s, rs) and gpu.equal(q, rq.view(gpu.uint8))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_special_rows(gpu, dtype):
