@@ -179,11 +179,12 @@ __global__ __launch_bounds__(kThreads) void k_quantize_rows(QuantArgs g) {
     for (int i = kCache * kThreads + (int)threadIdx.x; i < n; i += kThreads)
       store(load(i), i);
   } else {
-    for (int k = threadIdx.x; k < g.K; k += kThreads)
+    // (unsigned: K may lie within kThreads of 2^31)
+    for (unsigned k = threadIdx.x; k < (unsigned)g.K; k += kThreads)
       m = max(m, abs_bits(T::one(x + (long long)k * T::kBytes)));
     const float s = row_scale(block_max(m));
     if (threadIdx.x == 0) g.s[blockIdx.x] = s;
-    for (int k = threadIdx.x; k < g.K; k += kThreads) {
+    for (unsigned k = threadIdx.x; k < (unsigned)g.K; k += kThreads) {
       const float f = scaled(T::one(x + (long long)k * T::kBytes), s);
       q[k] = (uint8_t)pack_e4m3x4(f32x4{f, f, f, f});
     }

@@ -86,6 +86,23 @@ def test_more_rows_than_one_launch_has_workgroups(gpu, K):
 
 
 @pytest.mark.gpu
+def test_row_of_almost_2_31_elements(gpu):
+    """One row of 2^31 - 5 elements, read one by one: the index of a thread's
+    next element passes 2^31."""
+    K = 2 ** 31 - 5
+    say(f"case quantize M=1 K={K} bf16")
+    x = gpu.zeros((1, K), dtype=gpu.bfloat16, device="cuda")
+    at = gpu.tensor([0, 300, 2 ** 30, K - 300, K - 2, K - 1], device="cuda")
+    x[0, at] = gpu.tensor([1.0, -2, 3, -448, 28, 7], device="cuda", dtype=gpu.bfloat16)
+    q, s = entry(gpu, x)
+    gpu.cuda.synchronize()
+    assert s.item() == 1.0
+    want = gpu.tensor([1.0, -2, 3, -448, 28, 7], device="cuda").to(gpu.float8_e4m3fn)
+    assert gpu.equal(q[0, at], want.view(gpu.uint8))
+    assert int(gpu.count_nonzero(q)) == at.numel()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_special_rows(gpu, dtype):
     inf, nan = float("inf"), float("nan")
