@@ -156,15 +156,35 @@ def _plain_eager(x: torch.Tensor) -> bool:
             and x.device.index == torch.cuda.current_device())
 
 
+def _kernel_ahead(M: int, K: int, ld: int, size: int, ptr: int) -> bool:
+    """The kernel is faster than the tensor operations on M rows of K elements
+    of `size` bytes.  It gives each row a workgroup, so that it falls behind on
+    many rows of a few elements, where a workgroup has little to do, and on a
+    few very long rows, which leave CUs idle.  Measured against the operations
+    in a graph, which is where they are cheapest (us, kernel / operations):
+    bf16 65536x16 110 / 40, 65536x256 111 / 130, 16384x16 28 / 32; fp32
+    262144x64 207 / 164, x192 209 / 292; bf16 1x131072 30 / 35, 1x262144 60 /
+    36, 16x1048576 318 / 266, 256x1048576 604 / 1919; rows without 16-byte
+    loads: 262144x33 120 / 105, 1x16385 22 / 30, 1x65537 81 / 39, 256x65537 150
+    / 121, 1024x65537 172 / 464."""
+    if 256 <= K <= 20480:
+        return True
+    if (ptr | ld * size | K * size) % 16 == 0:
+        short, few, long, many = 512 // size, 8192 * size, (256 << 10) // size, 256
+    else:
+        short, few, long, many = 65, 65536, 20480, 1024
+    return (K >= short or M <= few) and (K <= long or M >= many)
+
+
 def quantize_rows(x: torch.Tensor):
     """Per-row e4m3 quantisation: returns (q, s) with q = x / s rounded to
     e4m3 (saturated to +-448) and s = amax(|row|) / 448 (float32, one per
     row; rows of zeros get s = 1).  x ~= q * s[:, None].
 
     Rows of float32, bfloat16 or float16 on the GPU go through one kernel
-    (hipgemm_quantize_rows_e4m3), with the same results bit for bit; under
-    autograd, a transform or a trace, on the CPU and for other layouts these
-    are tensor operations."""
+    (hipgemm_quantize_rows_e4m3) where that is faster (_kernel_ahead), with the
+    same results bit for bit; under autograd, a transform or a trace, on the CPU
+    and for other layouts these are tensor operations."""
     return _quantize_rows(x, _plain_eager(x))
 
 
@@ -173,7 +193,8 @@ def _quantize_rows(x: torch.Tensor, plain: bool):
     kind = _QUANT_TYPES.get(x.dtype)
     if plain and kind is not None and x.dim() == 2:
         (M, K), (ld, unit) = x.shape, x.stride()
-        if 0 < M < 2 ** 31 and 0 < K < 2 ** 31 and unit == 1 and ld >= K:
+        if (0 < M < 2 ** 31 and 0 < K < 2 ** 31 and unit == 1 and ld >= K
+                and _kernel_ahead(M, K, ld, x.element_size(), x.data_ptr())):
             dev = x.device
             q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=dev)
             s = torch.empty(M, dtype=torch.float32, device=dev)

@@ -85,6 +85,48 @@ def test_more_rows_than_one_launch_has_workgroups(gpu, K):
     assert gpu.equal(s, rs) and gpu.equal(q, rq.view(gpu.uint8))
 
 
+# (M, K, wide loads) -> whether the kernel takes it, for 2-byte elements.
+ROUTES = {(16384, 16, True): True, (16392, 16, True): False, (65536, 255, False): True,
+          (70000, 248, True): False, (70000, 256, True): True,
+          (65536, 3, False): True, (65544, 64, False): False, (65544, 65, False): True,
+          (1, 131072, True): True, (255, 131080, True): False, (256, 131080, True): True,
+          (1, 20481, False): False, (1023, 20481, False): False,
+          (1024, 20481, False): True, (1, 20480, False): True, (1, 256, False): True}
+
+
+def test_rows_the_kernel_takes():
+    """The choice by sizes, for 2- and 4-byte elements, and by alignment."""
+    for (M, K, wide), want in ROUTES.items():
+        assert ops._kernel_ahead(M, K, K, 2, 4096 if wide else 4098) is want, (M, K, wide)
+    assert ops._kernel_ahead(32768, 4, 4, 4, 4096)
+    assert not ops._kernel_ahead(32769, 124, 124, 4, 4096)
+    assert ops._kernel_ahead(32769, 128, 128, 4, 4096)
+    assert ops._kernel_ahead(1, 65536, 65536, 4, 4096)
+    assert not ops._kernel_ahead(1, 65540, 65540, 4, 4096)
+    assert not ops._kernel_ahead(1, 65536, 65537, 4, 4096)  # stride
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [s for s in ROUTES if s[0] * s[1] < 2 ** 25],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_kernel_where_it_is_ahead(gpu, monkeypatch, shape):
+    """Rows that the kernel is slower on are tensor operations, and the kernel's
+    results on them are theirs."""
+    M, K, wide = shape
+    say(f"case quantize route {M}x{K} wide={wide}")
+    x = gpu.randn((M, K + 8), device="cuda", dtype=gpu.bfloat16)
+    x = x[:, :K] if wide else x[:, 1:K + 1]
+    assert ((x.data_ptr() | 2 * x.stride(0) | 2 * K) % 16 == 0) == wide
+    q, s = entry(gpu, x)
+    rq, rs = ops._quantize_rows_ops(x)
+    assert gpu.equal(s, rs) and gpu.equal(q, rq.view(gpu.uint8))
+    calls = []
+    real = ops.lib
+    monkeypatch.setattr(ops, "lib", lambda: calls.append(1) or real())
+    ops.quantize_rows(x)
+    assert bool(calls) == ROUTES[shape]
+
+
 @pytest.mark.gpu
 def test_row_of_almost_2_31_elements(gpu):
     """One row of 2^31 - 5 elements, read one by one: the index of a thread's
