@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows,K", [(1, 32), (130, 256), (128, 288), (300, 2048),
                                     (257, 8192 + 32)])
 @pytest.mark.parametrize("pad,off,doff", [(0, 0, 0), (8, 8, 0), (3, 0, 0), (0, 1, 0),
-                                          (8, 0, 1), (5, 3, 7)])
+                                          (8, 0, 1), (5, 3, 7), (3, 4, 0), (7, 4, 16)])
 def test_pack_alignments(gpu, rows, K, pad, off, doff):
     torch = gpu
     say(f"case mx-pack rows={rows} K={K} ld=K/32+{pad} src+{off} dst+{doff}")
