@@ -708,7 +708,8 @@ size_t narrow_max_ws(int M, int N, int K, int variant) {
                                : variant_ws(M, N, K, variant);
 }
 
-// Workspace of an AUTO call that names `variant` and picked t (narrow).
+// Workspace of an AUTO call that names `variant` and picked t (narrow) with all
+// the workspace that it may take.
 size_t auto_ws(int M, int N, int K, int variant, int t, const NarrowPlan& narrow) {
   const size_t need = variant_ws(M, N, K, variant);
   return t == kTileNarrow && M <= CfgSkinny::kMaxM && narrow.ws_bytes > need
@@ -837,11 +838,12 @@ hipError_t run_gemm(const hipgemm_gemm_desc& d, bool ws_given,
   if (dry_run) return hipSuccess;
   if (d.variant == HIPGEMM_VARIANT_AUTO && fmt < 4 && !mx && K > 0) {
     NarrowPlan np;
-    const size_t max_ws = ws_given ? narrow_max_ws(M, N, K, variant) : 0;
+    // A workspace too small for the named schedule is refused whichever runs;
+    // AUTO's K-slices take no more than what is there.
+    if (ws_given && ws_bytes < variant_ws(M, N, K, variant)) return hipErrorInvalidValue;
+    const size_t most = narrow_max_ws(M, N, K, variant);
+    const size_t max_ws = !ws_given ? 0 : ws_bytes < most ? ws_bytes : most;
     int t = pick_tile(M, N, K, cu_count(), max_ws, &np);
-    // A workspace too small for what hipgemm_workspace_size names is refused
-    // whichever schedule runs.
-    if (ws_given && ws_bytes < auto_ws(M, N, K, variant, t, np)) return hipErrorInvalidValue;
     // fp32 and e4m3 outputs are not built for the 64-column K-slices.
     if (t == kTileNarrow && np.slices > 1 && key.out >= kOutF32)
       t = pick_tile(M, N, K, cu_count(), 0, &np);

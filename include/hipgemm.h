@@ -240,7 +240,9 @@ hipError_t hipgemm_fp8_gemm_bf16(const void *A, const void *B_T, void *C,
  * HIPGEMM_WS_COUNTER_BYTES bytes zero before its first use (every call
  * leaves them zero: see HIPGEMM_WS_COUNTER_BYTES).  Calls that may run
  * concurrently must not share a workspace.  Returns hipErrorInvalidValue if
- * it is missing or too small when needed.
+ * it is missing or too small when needed.  It is not needed for AUTO's
+ * 64-column tiles (hipgemm_auto_tile): where only their K-slices would use it,
+ * a call with less, or none, runs them in the slices that fit, or over whole K.
  * While `stream` is being captured into a graph, an entry point given no
  * workspace allocates none: a schedule that would split K runs with one
  * K-slice (the same result within rounding, slower on the shapes that
@@ -392,9 +394,9 @@ int hipgemm_split_columns(int M, int N, int K);
  * calls run the 128 x 128 schedule's pipeline in one launch on 128 x 256, 192
  * x 192, 192 x 128 or 128 x 128 tiles (above 128 rows, no workspace) or, up to
  * 1024 rows, on 128 x 64 or 64 x 64 tiles -- those in K-slices where that is
- * faster and the call brings the workspace hipgemm_workspace_size names for
- * AUTO (or runs hipgemm_gemm_noalloc), the last slice to arrive at a part of a
- * tile summing it.  No reference counterpart (the reference has 256 x 256
+ * faster and the call brings a workspace that holds them (what
+ * hipgemm_workspace_size names for AUTO does) or runs hipgemm_gemm_noalloc, the
+ * last slice to arrive at a part of a tile summing it.  No reference counterpart (the reference has 256 x 256
  * tiles only). */
 int hipgemm_auto_tile(int M, int N, int K, int *bm, int *bn);
 

@@ -64,8 +64,9 @@ def test_auto_tile_keeps_other_choices():
 
 
 def test_short_workspace_is_refused():
-    """Whichever tile runs, AUTO refuses a workspace below
-    hipgemm_workspace_size (before any launch)."""
+    """Whichever tile runs, AUTO refuses a workspace too small for the schedule
+    that hipgemm_select_variant names (before any launch); in these shapes that
+    schedule needs all of hipgemm_workspace_size."""
     fake = 1 << 20
     for M, N, K in SHAPES:
         need = hg.workspace_size(M, N, K, 0)

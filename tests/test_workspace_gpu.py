@@ -12,6 +12,8 @@ HIPGEMM_WS_COUNTER_BYTES) and of graph capture around it.
   instead of recording an allocation and a memset into the caller's graph:
   the 128 x 128 schedule's K-slices at 256 x 8192 x 8192 and the strip
   schedule's at 16 x 4096 x 4096; every replay equals the oracle.
+* Where only AUTO's 64-column K-slices would use a workspace, a call with a
+  smaller one or none runs.
 """
 import numpy as np
 import pytest
@@ -134,3 +136,28 @@ def test_capture_without_workspace_runs_unsplit(gpu, oracle, M, N, K):
             say(f"    replay {r} output {i}: "
                 f"{int((got != want).sum())} of {M * N} differ")
             assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 8192, 4096), (33, 4608, 4096)])
+def test_workspace_of_optional_slices(gpu, oracle, M, N, K):
+    """AUTO names the strip schedule in one K-slice here and runs 64-column
+    tiles: in K-slices with the workspace that hipgemm_workspace_size names,
+    over whole K with 256 bytes less or with none."""
+    torch = gpu
+    need = hg.workspace_size(M, N, K, 0)
+    assert hg.select_variant(M, N, K) == hg.VARIANTS["strip"] and need > 16384
+    assert hg.auto_tile(M, N, K)[1] == 64
+    A, B = ternary((M, K), 97), ternary((N, K), 98)
+    a, b = to_dev(torch, A), to_dev(torch, B)
+    want = oracle.gemm(A, B)
+    ws = torch.zeros(need, dtype=torch.uint8, device="cuda")
+    for nbytes in (need, need - 256, 16384 + 256, 16384, 0):
+        say(f"case optional workspace {M}x{N}x{K}: {nbytes} of {need} bytes")
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        assert hg.gemm_raw_ws(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, K, K, N,
+                              0, 0, 0, ws.data_ptr() if nbytes else 0, nbytes,
+                              torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(from_dev_bf16(c), want)
+        assert bool(ws[nbytes:].eq(0).all()) and bool(ws[:16384].eq(0).all())
+        ws.zero_()
