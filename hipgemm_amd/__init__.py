@@ -382,19 +382,20 @@ def _mx_ptr(t, rows, K, name):
     return t.data_ptr()
 
 
-# Workspace bytes by sizes and options (a pure function of them on one GPU
-# model; the C call and a descriptor cost 2 us per GEMM).
+# Workspace bytes by sizes and options, and how many of them the call has to
+# have: the rest is for K-slices that AUTO can do without, which fp32 outputs
+# never take (a pure function of them on one GPU model; the C calls and
+# descriptors cost 2 us per GEMM).
 @functools.lru_cache(maxsize=4096)
 def _ws_bytes(device: int, M: int, N: int, K: int, variant: int,
               a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
-              mx: bool = False) -> int:
-    if M <= 0 or N <= 0:
-        return 0
-    if not mx and a_format <= FMT_E5M2 and b_format <= FMT_E5M2:
-        return workspace_size(M, N, K, variant)
-    d = GemmDesc(M=M, N=N, K=K, a_format=a_format, b_format=b_format,
-                 variant=variant, mx_scale_a=int(mx), mx_scale_b=int(mx))
-    return int(lib().hipgemm_gemm_workspace_size(ctypes.byref(d)))
+              mx: bool = False, out: int = OUT_BF16):
+    def need(out_dtype):
+        d = GemmDesc(M=M, N=N, K=K, a_format=a_format, b_format=b_format,
+                     out_dtype=out_dtype, variant=variant, mx_scale_a=int(mx),
+                     mx_scale_b=int(mx))
+        return int(lib().hipgemm_gemm_workspace_size(ctypes.byref(d)))
+    return need(out), need(OUT_F32)
 
 
 def _gemm_operands(a, b_t, out, stream, out_dtype=None):
@@ -508,7 +509,8 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     so = _scale_ptr(scale_out, "scale_out")
     ws, nbytes = _stream_workspace(
         a, stream, handle, _ws_bytes(a.get_device(), M, N, K, variant, a_format,
-                                     b_format, bool(mx_a or mx_b)))
+                                     b_format, bool(mx_a or mx_b),
+                                     codes[out_dtype]))
     d = _Desc(_DESC_BYTES, a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
               lda, ldb, ldc, a_format, b_format, codes[out_dtype],
               ACTIVATIONS[activation], *ptrs, variant, ws, nbytes, mx_a, mx_b, so)
@@ -564,10 +566,15 @@ _workspaces: dict = {}
 _retired: list = []
 
 
-def _stream_workspace(a, stream, handle: int, nbytes: int):
-    """(pointer, nbytes) of the workspace of a's device and `stream` (None: the
-    current one; `handle` is its handle), or (0, 0) where none is needed or
-    none may be allocated."""
+def _stream_workspace(a, stream, handle: int, need):
+    """(pointer, bytes) of the workspace of a's device and `stream` (None: the
+    current one; `handle` is its handle) for a call with `need` of _ws_bytes, or
+    (0, 0) where none is needed or none may be allocated."""
+    nbytes, required = need
+    # A graph keeps only the workspace it has to have: replayed on another
+    # stream, it shares that with this stream's calls.
+    if nbytes > required and _capturing(a, stream):
+        nbytes = required
     if not nbytes:
         return 0, 0
     ws = _workspaces.get((a.get_device(), handle))
@@ -580,6 +587,18 @@ def _stream_workspace(a, stream, handle: int, nbytes: int):
     return ws.data_ptr(), nbytes
 
 
+def _capturing(a, stream) -> bool:
+    """Whether `stream` itself (it need not be the current one; None: the current
+    one of a's device) is being captured."""
+    cuda = _torch().cuda
+    if stream is None:
+        if a.get_device() == cuda.current_device():
+            return cuda.is_current_stream_capturing()
+        stream = cuda.current_stream(a.device)
+    with cuda.stream(stream):
+        return cuda.is_current_stream_capturing()
+
+
 def _workspace(device, stream, nbytes: int):
     """The stream's workspace of at least nbytes, or None while `stream` is
     being captured and has none that large."""
@@ -587,11 +606,7 @@ def _workspace(device, stream, nbytes: int):
     key = (device.index, stream.cuda_stream)
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
-        # The capture status of `stream` itself (it need not be the current
-        # stream).
-        with torch.cuda.stream(stream):
-            capturing = torch.cuda.is_current_stream_capturing()
-        if capturing:
+        if _capturing(None, stream):
             return None
         size = nbytes if ws is None else max(nbytes, 2 * ws.numel())
         with torch.cuda.stream(stream):

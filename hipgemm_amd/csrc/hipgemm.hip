@@ -989,6 +989,40 @@ int fp4_variant(int variant, int M, int N, int Kb) {
              : HIPGEMM_VARIANT_TILE128;
 }
 
+// Workspace bytes of a descriptor's call; slices: with what AUTO's 64-column
+// K-slices may take beyond what the call has to have.
+size_t desc_ws(const hipgemm_gemm_desc* d, bool slices) {
+  if (!d || d->size != sizeof(hipgemm_gemm_desc) || d->M <= 0 || d->N <= 0 ||
+      d->K <= 0)
+    return 0;
+  const bool fp4 = d->a_format == HIPGEMM_FMT_FP4_E2M1 ||
+                   d->b_format == HIPGEMM_FMT_FP4_E2M1;
+  if (fp4) {
+    if (fp4_variant(d->variant, d->M, d->N, d->K / 2) == HIPGEMM_VARIANT_4WAVE_MFMA16)
+      return 0;
+    return plan_t128(d->M, d->N, d->K / 2, cu_count()).ws_bytes;
+  }
+  auto is6 = [](int f) {
+    return f == HIPGEMM_FMT_FP6_E2M3 || f == HIPGEMM_FMT_FP6_E3M2;
+  };
+  const bool fp6 = is6(d->a_format) || is6(d->b_format);
+  if (fp6) {
+    if (fp4_variant(d->variant, d->M, d->N, d->K / 4 * 3) ==
+        HIPGEMM_VARIANT_4WAVE_MFMA16)
+      return 0;
+    return plan_t128(d->M, d->N, d->K / 4 * 3, cu_count(), 96).ws_bytes;
+  }
+  if (d->mx_scale_a || d->mx_scale_b) {  // 128 x 128 where AUTO picks it
+    const int v = resolve_variant(d->variant, d->M, d->N, d->K);
+    return v == HIPGEMM_VARIANT_TILE128
+               ? plan_t128(d->M, d->N, d->K, cu_count()).ws_bytes
+               : 0;
+  }
+  // fp32 and e4m3 outputs are not built for the 64-column K-slices.
+  if (slices && d->out_dtype < HIPGEMM_OUT_F32)
+    return hipgemm_workspace_size(d->M, d->N, d->K, d->variant);
+  return variant_ws(d->M, d->N, d->K, resolve_variant(d->variant, d->M, d->N, d->K));
+}
 
 }  // namespace
 
@@ -1186,33 +1220,7 @@ hipError_t hipgemm_quantize_rows_e4m3(const void* x, int type, int M, int K,
 }
 
 size_t hipgemm_gemm_workspace_size(const hipgemm_gemm_desc* d) {
-  if (!d || d->size != sizeof(hipgemm_gemm_desc) || d->M <= 0 || d->N <= 0 ||
-      d->K <= 0)
-    return 0;
-  const bool fp4 = d->a_format == HIPGEMM_FMT_FP4_E2M1 ||
-                   d->b_format == HIPGEMM_FMT_FP4_E2M1;
-  if (fp4) {
-    if (fp4_variant(d->variant, d->M, d->N, d->K / 2) == HIPGEMM_VARIANT_4WAVE_MFMA16)
-      return 0;
-    return plan_t128(d->M, d->N, d->K / 2, cu_count()).ws_bytes;
-  }
-  auto is6 = [](int f) {
-    return f == HIPGEMM_FMT_FP6_E2M3 || f == HIPGEMM_FMT_FP6_E3M2;
-  };
-  const bool fp6 = is6(d->a_format) || is6(d->b_format);
-  if (fp6) {
-    if (fp4_variant(d->variant, d->M, d->N, d->K / 4 * 3) ==
-        HIPGEMM_VARIANT_4WAVE_MFMA16)
-      return 0;
-    return plan_t128(d->M, d->N, d->K / 4 * 3, cu_count(), 96).ws_bytes;
-  }
-  if (d->mx_scale_a || d->mx_scale_b) {  // 128 x 128 where AUTO picks it
-    const int v = resolve_variant(d->variant, d->M, d->N, d->K);
-    return v == HIPGEMM_VARIANT_TILE128
-               ? plan_t128(d->M, d->N, d->K, cu_count()).ws_bytes
-               : 0;
-  }
-  return hipgemm_workspace_size(d->M, d->N, d->K, d->variant);
+  return desc_ws(d, true);
 }
 
 hipError_t hipgemm_gemm_noalloc(const hipgemm_gemm_desc* desc,
@@ -1220,7 +1228,9 @@ hipError_t hipgemm_gemm_noalloc(const hipgemm_gemm_desc* desc,
   if (!desc || desc->size != sizeof(hipgemm_gemm_desc) || desc->workspace ||
       desc->workspace_bytes)
     return hipErrorInvalidValue;
-  const size_t need = hipgemm_gemm_workspace_size(desc);
+  // Not for K-slices alone that the call can do without: calls that need no
+  // scratch stay independent of those that share it.
+  const size_t need = desc_ws(desc, false);
   if (need > (size_t)HIPGEMM_NOALLOC_SCRATCH_BYTES) return hipErrorInvalidValue;
   hipgemm_gemm_desc d = *desc;
   if (need > 0) {
@@ -1231,8 +1241,8 @@ hipError_t hipgemm_gemm_noalloc(const hipgemm_gemm_desc* desc,
     if (!d.workspace) return e;
     d.workspace_bytes = HIPGEMM_NOALLOC_SCRATCH_BYTES;
   }
-  // need == 0: no schedule on this path uses a workspace (none is given,
-  // so none can be allocated either).
+  // need == 0: no schedule on this path needs a workspace (none is given, so
+  // none is used or allocated).
   return run_gemm(d, true, stream);
 }
 

@@ -306,7 +306,9 @@ hipError_t hipgemm_gemm(const hipgemm_gemm_desc *desc, hipStream_t stream);
  * its own translation unit, which the HIP runtime loads on a GPU at the first
  * hipgemm_gemm_noalloc call there that needs scratch, and holds until the
  * process ends (with the runtime's deferred code-object loading; without
- * it, on every GPU where the library's code is loaded).  No call makes an
+ * it, on every GPU where the library's code is loaded).  AUTO's 64-column
+ * K-slices use it too, but do not make a call need it (they run over whole K
+ * where nothing else of the call would).  No call makes an
  * allocation or a memset.
  * desc->workspace must be NULL and desc->workspace_bytes 0.  Returns
  * hipErrorInvalidValue when the descriptor is invalid (as hipgemm_gemm) or
@@ -361,7 +363,7 @@ size_t hipgemm_workspace_size(int M, int N, int K, int variant);
 
 /* Workspace bytes hipgemm_gemm needs for this descriptor on the current
  * device (0: none, or an invalid descriptor); it accounts for the operand
- * formats and the schedule AUTO takes for them.  No GPU work.  No reference
+ * formats, the output type and the schedule AUTO takes for them.  No GPU work.  No reference
  * counterpart. */
 size_t hipgemm_gemm_workspace_size(const hipgemm_gemm_desc *desc);
 

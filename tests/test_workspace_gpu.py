@@ -13,8 +13,11 @@ HIPGEMM_WS_COUNTER_BYTES) and of graph capture around it.
   the 128 x 128 schedule's K-slices at 256 x 8192 x 8192 and the strip
   schedule's at 16 x 4096 x 4096; every replay equals the oracle.
 * Where only AUTO's 64-column K-slices would use a workspace, a call with a
-  smaller one or none runs.
+  smaller one or none runs, and neither hipgemm_gemm_noalloc nor a graph that
+  the Python helpers capture shares scratch memory for them.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -161,3 +164,45 @@ def test_workspace_of_optional_slices(gpu, oracle, M, N, K):
         assert np.array_equal(from_dev_bf16(c), want)
         assert bool(ws[nbytes:].eq(0).all()) and bool(ws[:16384].eq(0).all())
         ws.zero_()
+
+
+def test_optional_slices_share_no_scratch(gpu):
+    """hipgemm_gemm_noalloc's calls and captured graphs stay independent of others
+    where the schedule that AUTO names needs no scratch: they run over whole K,
+    as a call without a workspace does.  The fp32 sums tell (whole K and
+    K-slices differ in a few of 2^19 outputs)."""
+    torch = gpu
+    M, N, K = 64, 8192, 4096
+    say(f"case optional slices share no scratch {M}x{N}x{K}")
+    rng = np.random.default_rng(31)  # every finite e4m3 value: inexact sums
+    A, B = (rng.integers(0, 127, shape, np.uint8) | rng.integers(0, 2, shape, np.uint8) << 7
+            for shape in ((M, K), (N, K)))
+    a, b = to_dev(torch, A), to_dev(torch, B)
+    c = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    d = hg.GemmDesc(A=a.data_ptr(), B_T=b.data_ptr(), C=c.data_ptr(), M=M, N=N, K=K,
+                    lda=K, ldb=K, ldc=N)
+
+    def result(code):
+        assert code == 0
+        torch.cuda.synchronize()
+        return from_dev_bf16(c).copy()
+    cur = torch.cuda.current_stream().cuda_stream
+    whole = result(hg.gemm_desc_raw(d, cur))
+    assert np.array_equal(result(hg.gemm_desc_noalloc_raw(d, cur)), whole)
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        sliced = from_dev_bf16(hg.fp8_gemm_bf16(a, b))
+    s.synchronize()
+    assert hg._workspaces[(0, s.cuda_stream)].numel() >= hg.workspace_size(M, N, K, 0) > 0
+    assert 0 < int((sliced != whole).sum()) < M * N // 100
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        hg.gemm(a, b, out=c)
+    for _ in range(3):
+        c.fill_(float("nan"))
+        graph.replay()
+        assert np.array_equal(result(0), whole)
+    # fp32 outputs take no slices: their query names none.
+    d.out_dtype = hg.OUT_F32
+    assert hg.lib().hipgemm_gemm_workspace_size(ctypes.addressof(d)) == 0
