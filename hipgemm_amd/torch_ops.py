@@ -166,9 +166,7 @@ def _kernel_ahead(M: int, K: int, ld: int, size: int, ptr: int) -> bool:
     262144x64 207 / 164, x192 209 / 292; bf16 1x131072 30 / 35, 1x262144 60 /
     36, 16x1048576 318 / 266, 256x1048576 604 / 1919; rows without 16-byte
     loads: 262144x33 120 / 105, 1x16385 22 / 30, 1x65537 81 / 39, 256x65537 150
-    / 121, 1024x65537 172 / 464."""
-    if 256 <= K <= 20480:
-        return True
+    / 121, 1024x65537 172 / 464.  (At 256 to 20480 elements always.)"""
     if (ptr | ld * size | K * size) % 16 == 0:
         short, few, long, many = 512 // size, 8192 * size, (256 << 10) // size, 256
     else:
@@ -194,7 +192,8 @@ def _quantize_rows(x: torch.Tensor, plain: bool):
     if plain and kind is not None and x.dim() == 2:
         (M, K), (ld, unit) = x.shape, x.stride()
         if (0 < M < 2 ** 31 and 0 < K < 2 ** 31 and unit == 1 and ld >= K
-                and _kernel_ahead(M, K, ld, x.element_size(), x.data_ptr())):
+                and (256 <= K <= 20480
+                     or _kernel_ahead(M, K, ld, x.element_size(), x.data_ptr()))):
             dev = x.device
             q = torch.empty((M, K), dtype=torch.float8_e4m3fn, device=dev)
             s = torch.empty(M, dtype=torch.float32, device=dev)
