@@ -174,8 +174,11 @@ hipError_t launch_tile(int t, const void* fn, GemmArgs g, hipStream_t stream) {
 
 // 64-column tiles on plan p; nullptr where they are not built for the call.
 const void* narrow_kernel(const NarrowPlan& p, const GemmArgs& g, hk::Key* key) {
+  // B_T read once: where its rows are whole 128-byte lines, so that no step
+  // shares one with the next (the hint would have it fetched twice).
+  const bool lines = g.ldb % 128 == 0 && aligned(g.B, 128);
   const int mode = p.slices > 1 ? hk::kNarrowSplit
-                   : g.M <= hk::kNarrow[p.tile].bm ? hk::kNarrowOnce
+                   : lines && g.M <= hk::kNarrow[p.tile].bm ? hk::kNarrowOnce
                                                    : hk::kNarrowWhole;
   key->vec = vec_ok(key->out, g.N, g.ldc, g.C, key->out >= kOutF32 ? 4 : 8);
   return !key->ext            ? hk::narrow_plain(p.tile, mode, *key)

@@ -74,7 +74,9 @@
 // kNt: B_T's DMA carry the non-temporal hint, for one row of tiles, where each
 // B_T line is read by one workgroup (64 x 14336 x 4096 on 64 x 64 tiles 14.9 ->
 // 13.8 us, 128 x 14336 x 4096 18.5 -> 17.7; with K-slices level to 10 %
-// slower).
+// slower), in one step: with rows that do not start on 128-byte lines each line
+// belongs to two steps, and the hint cost 8 % at the median of 167 such shapes
+// (30 % at most).
 //
 // kMx: MX block scales from g.mx (the packed layout of MxArgs; per-tensor
 // epilogue).  Each step also loads, two steps ahead, each operand's 16 scale
