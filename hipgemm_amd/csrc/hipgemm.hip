@@ -566,8 +566,8 @@ double tile_cost(const TileCost& c, int M, int N, int K, int cus) {
 // Cost of what hipgemm_select_variant and hipgemm_split_columns name for 33
 // rows and more (the same model; the strip's per step the bytes of its columns
 // and of A's row blocks; 5-7 % standard error on 146 and 135 shapes up to 128
-// rows).
-double named_cost(int M, int N, int K, int cus) {
+// rows).  ws: the call brings the schedule's workspace.
+double named_cost(int M, int N, int K, int cus, bool ws) {
   const int variant = hipgemm_select_variant(M, N, K);
   if (variant == HIPGEMM_VARIANT_STRIP) {
     const StripPlan p = plan_strip(M, N, K, strip_knb(M, N, K));
@@ -576,8 +576,18 @@ double named_cost(int M, int N, int K, int cus) {
     return 3.54 + p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) + 1.10 * area +
            (p.slices > 1 ? 2.02 + 0.189 * p.slices * area : 0.0);
   }
-  // The split-K schedule: never ahead of 64-column tiles where it is named.
-  if (variant == HIPGEMM_VARIANT_SKINNY) return 1e9;
+  // The split-K schedule (9 % standard error on 300 shapes): always behind
+  // 64-column tiles in K-slices, but ahead of whole K, which fp32 and e4m3
+  // outputs take, on few columns of long rows: fp32 128 x 2048 x 8192 15.4
+  // against 20.4 us, 120 x 2048 x 10112 18.3 / 24.5; 79 x 2560 x 4096 14.4 /
+  // 10.5.  Without a workspace it would allocate one (22 us and more) or, under
+  // capture, not split.
+  if (variant == HIPGEMM_VARIANT_SKINNY) {
+    if (!ws) return 1e9;
+    const SkinnyPlan p = plan_skinny(M, N, K);
+    const int units = p.tiles_n * p.slices;
+    return 7.9 + 0.57 * ceil_div(units, cus) * p.slice_steps * p.bn / 128 + 5.3 * units / cus;
+  }
   const int n1 = split_columns(M, N, cus);
   if (n1 > 0)
     return 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus) +
@@ -662,11 +672,12 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm) 
 //    least certain; 320 shapes up to 1024 rows: 11 % faster on average, 13 %
 //    slower at worst), else 5 %.  Up to 32 rows the strip, which reads A into
 //    registers, stays ahead.
-// max_ws: workspace bytes that K-slices may take (0: none).
+// ws: the call brings a workspace.  max_ws: the bytes of it that K-slices may
+// take (0: none).
 constexpr int kNoTile = -1, kTile128 = -2, kTileNarrow = -3;
-int pick_tile(int M, int N, int K, int cus, size_t max_ws, NarrowPlan* narrow) {
+int pick_tile(int M, int N, int K, int cus, bool ws, size_t max_ws, NarrowPlan* narrow) {
   if (M <= 32 || K <= 0 || N <= 0) return kNoTile;
-  const double named = named_cost(M, N, K, cus);
+  const double named = named_cost(M, N, K, cus, ws);
   int best = kNoTile;
   double cost = named;
   if (M > CfgSkinny::kMaxM) {
@@ -846,10 +857,10 @@ hipError_t run_gemm(const hipgemm_gemm_desc& d, bool ws_given,
     if (ws_given && ws_bytes < variant_ws(M, N, K, variant)) return hipErrorInvalidValue;
     const size_t most = narrow_max_ws(M, N, K, variant);
     const size_t max_ws = !ws_given ? 0 : ws_bytes < most ? ws_bytes : most;
-    int t = pick_tile(M, N, K, cu_count(), max_ws, &np);
+    int t = pick_tile(M, N, K, cu_count(), ws_given, max_ws, &np);
     // fp32 and e4m3 outputs are not built for the 64-column K-slices.
     if (t == kTileNarrow && np.slices > 1 && key.out >= kOutF32)
-      t = pick_tile(M, N, K, cu_count(), 0, &np);
+      t = pick_tile(M, N, K, cu_count(), ws_given, 0, &np);
     // The tiles are not built for every epilogue: else what follows.
     hk::Key k = key;
     const void* fn = nullptr;
@@ -1130,14 +1141,14 @@ int hipgemm_split_columns(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int cus = cu_count();
   NarrowPlan np;
-  return pick_tile(M, N, K, cus, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
+  return pick_tile(M, N, K, cus, false, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
 }
 
 int hipgemm_auto_tile(int M, int N, int K, int* bm, int* bn) {
   if (!bm || !bn) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   NarrowPlan np;
-  const int t = pick_tile(M, N, K, cu_count(),
+  const int t = pick_tile(M, N, K, cu_count(), true,
                           narrow_max_ws(M, N, K, hipgemm_select_variant(M, N, K)), &np);
   if (t == kNoTile) return 0;
   const hk::TileShape s = t == kTileNarrow ? hk::kNarrow[np.tile]
@@ -1256,7 +1267,7 @@ size_t hipgemm_workspace_size(int M, int N, int K, int variant) {
   if (v != named || K == 0) return variant_ws(M, N, K, v);
   // The schedule AUTO names covers AUTO's 64-column K-slices too.
   NarrowPlan np;
-  const int t = pick_tile(M, N, K, cu_count(), narrow_max_ws(M, N, K, v), &np);
+  const int t = pick_tile(M, N, K, cu_count(), true, narrow_max_ws(M, N, K, v), &np);
   return auto_ws(M, N, K, v, t, np);
 }
 

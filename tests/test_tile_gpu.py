@@ -169,3 +169,25 @@ def test_each_xcd_starts_at_its_own_step(gpu, tail):
     assert np.all(tiles == sums[None, :, None])
     assert np.all((sums >= 2.0 ** 23) & (sums <= 2.0 ** 23 + 4)), sums
     assert len(set(sums)) > 1, sums
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,split", [((128, 2048, 8192), True),
+                                         ((79, 2560, 4096), False)])
+def test_split_k_where_outputs_take_no_slices(gpu, shape, split):
+    """AUTO names the split-K schedule at both shapes.  bf16 outputs run K-slices
+    of 64-column tiles; fp32 outputs, which have none, run the schedule itself
+    or whole K, whichever is faster.  The fp32 sums tell which ran (their results are
+    checked where sums are exact)."""
+    torch = gpu
+    M, N, K = shape
+    say(f"case split-K or whole K M={M} N={N} K={K} fp32 output")
+    skinny = hg.VARIANTS["skinny"]
+    assert hg.select_variant(M, N, K) == skinny and hg.auto_tile(M, N, K)[1] == 64
+    rng = np.random.default_rng(8)  # every finite e4m3 value: inexact sums
+    a, b = (to_dev(torch, rng.integers(0, 127, s, np.uint8) |
+                   rng.integers(0, 2, s, np.uint8) << 7) for s in ((M, K), (N, K)))
+    f32 = torch.float32
+    auto = hg.gemm(a, b, out_dtype=f32)
+    named = hg.gemm(a, b, out_dtype=f32, variant=skinny)
+    assert torch.equal(auto, named) == split
