@@ -547,33 +547,43 @@ int split_columns(int M, int N, int cus) {
 // epilogue) and per launch.  Fitted to 298 shapes (129 to 8192 rows, N 1024 to
 // 28672, K 512 to 14336; half of them a grid of usual sizes, half random),
 // every tile timed on each: 5-9 % standard error per tile.
+// ragged: how much longer the steps take where rows do not start on 128-byte
+// lines, so that a step's part of a row lies in two.  These factors and the ones
+// below come from 1100 such shapes from 33 rows up, operands from memory: without
+// them 97 of 2100 choices were more than 3 % behind the named schedule (64 x 64
+// tiles, 55 x 16472 x 13744 106 against 86 us), with them 42, and all together
+// 1.0 % behind the fastest instead of 1.25.
 struct TileCost {
   int bm, bn;
-  double launch, round, step, busy;
+  double launch, round, step, busy, ragged;
 };
-constexpr TileCost kCost256{256, 256, 0.99, 6.86, 0.847, 0.370};
-constexpr TileCost kCost128{128, 128, 3.15, 1.23, 0.309, 0.149};
-constexpr TileCost kCostMid[hk::kNumTiles] = {{128, 256, 2.91, 2.57, 0.496, 0.248},
-                                              {192, 192, 2.92, 3.35, 0.507, 0.280},
-                                              {192, 128, 2.54, 2.15, 0.369, 0.213}};
-double tile_cost(const TileCost& c, int M, int N, int K, int cus) {
+constexpr TileCost kCost256{256, 256, 0.99, 6.86, 0.847, 0.370, 1.15};
+constexpr TileCost kCost128{128, 128, 3.15, 1.23, 0.309, 0.149, 1.28};
+constexpr TileCost kCostMid[hk::kNumTiles] = {{128, 256, 2.91, 2.57, 0.496, 0.248, 1.22},
+                                              {192, 192, 2.92, 3.35, 0.507, 0.280, 1.22},
+                                              {192, 128, 2.54, 2.15, 0.369, 0.213, 1.22}};
+// lines: the rows of A and B_T start on 128-byte lines.
+double tile_cost(const TileCost& c, int M, int N, int K, int cus, bool lines) {
   const int tiles = ceil_div(M, c.bm) * ceil_div(N, c.bn);
   const int rounds = ceil_div(tiles, cus);
   return c.launch + c.round * rounds +
-         ceil_div(K, 128) * (c.step * rounds + c.busy * tiles / cus);
+         (lines ? 1.0 : c.ragged) * ceil_div(K, 128) *
+             (c.step * rounds + c.busy * tiles / cus);
 }
 
 // Cost of what hipgemm_select_variant and hipgemm_split_columns name for 33
 // rows and more (the same model; the strip's per step the bytes of its columns
 // and of A's row blocks; 5-7 % standard error on 146 and 135 shapes up to 128
-// rows).  ws: the call brings the schedule's workspace.
-double named_cost(int M, int N, int K, int cus, bool ws) {
+// rows).  ws: the call brings the schedule's workspace; lines: as above.
+double named_cost(int M, int N, int K, int cus, bool ws, bool lines) {
   const int variant = hipgemm_select_variant(M, N, K);
   if (variant == HIPGEMM_VARIANT_STRIP) {
     const StripPlan p = plan_strip(M, N, K, strip_knb(M, N, K));
     const double w = p.knb / 2.0, area = p.kmb * p.knb / 8.0;
     const int rounds = ceil_div(p.tiles_n * p.slices, cus);
-    return 3.54 + p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) + 1.10 * area +
+    return 3.54 +
+           (lines ? 1.0 : 1.27) * p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) +
+           1.10 * area +
            (p.slices > 1 ? 2.02 + 0.189 * p.slices * area : 0.0);
   }
   // The split-K schedule (9 % standard error on 300 shapes): always behind
@@ -590,19 +600,23 @@ double named_cost(int M, int N, int K, int cus, bool ws) {
   }
   const int n1 = split_columns(M, N, cus);
   if (n1 > 0)
-    return 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus) +
-           0.91 * tile_cost(kCost128, M, N - n1, K, cus);
-  if (variant != HIPGEMM_VARIANT_TILE128) return tile_cost(kCost256, M, N, K, cus);
+    return 0.46 + 1.02 * tile_cost(kCost256, M, n1, K, cus, lines) +
+           0.91 * tile_cost(kCost128, M, N - n1, K, cus, lines);
+  if (variant != HIPGEMM_VARIANT_TILE128)
+    return tile_cost(kCost256, M, N, K, cus, lines);
+  const double f = lines ? 1.0 : 1.14;
   const T128Plan ks = plan_t128(M, N, K, cus);
   const double units = (double)ceil_div(M, 128) * ceil_div(N, 128) * ks.slices / cus;
   if (M <= CfgSkinny::kMaxM) {
-    const double c = 3.81 + ks.slice_steps * (0.375 * ceil_div((int)(units * cus), cus) + 0.326 * units) +
+    const double c = 3.81 +
+                     f * ks.slice_steps *
+                         (0.375 * ceil_div((int)(units * cus), cus) + 0.326 * units) +
                      (ks.slices > 1 ? 3.36 + 3.82 * units + 0.07 * (ks.slices - 1) : 0.0);
-    const double hbm = 3.0 + (double)N * K / 5.4e6;  // B_T at 5.4 TB/s
+    const double hbm = 3.0 + f * N * K / 5.4e6;  // B_T at 5.4 TB/s
     return c > hbm ? c : hbm;
   }
-  return ks.slices > 1 ? 9.64 + ks.slice_steps * (0.207 + 0.073 * units) + 6.01 * units
-                       : tile_cost(kCost128, M, N, K, cus);
+  return ks.slices > 1 ? 9.64 + f * ks.slice_steps * (0.207 + 0.073 * units) + 6.01 * units
+                       : tile_cost(kCost128, M, N, K, cus, lines);
 }
 
 // 64-column tiles (hk::kNarrow) in `slices` K-slices: a stream over B_T for
@@ -625,10 +639,13 @@ constexpr NarrowCost kNarrowFew[hk::kNumNarrow] = {
 constexpr NarrowCost kNarrowMany[hk::kNumNarrow] = {
     {3.04, 0.89, 0.236, 0.119, 0.68, 2.77, 0.787},
     {2.92, 0.82, 0.156, 0.075, 0.96, 1.04, 0.607}};
+// As TileCost::ragged, over whole K and in slices.
+constexpr double kNarrowRagged = 1.20, kSlicesRagged = 1.10;
 // The cheapest plan: K-slices of at least 8 steps, at most one workgroup per
 // CU, within max_ws bytes of workspace.  hbm: bytes per us that a stream of B_T
 // under one row of tiles reaches.
-NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm) {
+NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm,
+                       bool lines) {
   NarrowPlan best;
   const int steps = ceil_div(K, 128);
   for (int t = 0; t < hk::kNumNarrow; ++t) {
@@ -643,14 +660,16 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm) 
       p.slices = ceil_div(steps, p.slice_steps);
       const int units = tiles * p.slices, rounds = ceil_div(units, cus);
       const double share = (double)units / cus;
-      p.cost = c.launch + c.round * rounds + p.slice_steps * (c.step * rounds + c.busy * share);
+      const double f = lines ? 1.0 : p.slices > 1 ? kSlicesRagged : kNarrowRagged;
+      p.cost = c.launch + c.round * rounds +
+               f * p.slice_steps * (c.step * rounds + c.busy * share);
       if (p.slices > 1) {
         p.cost += c.split + c.units * share + c.slice * (p.slices - 1);
         p.ws_bytes = kWsCounterBytes +
                      (size_t)units * hk::kNarrow[t].bm * hk::kNarrow[t].bn * sizeof(float);
         if (p.ws_bytes > max_ws || 4 * tiles > kWsMaxCounters) continue;
       }
-      if (few && p.cost < 3.0 + (double)N * K / hbm) p.cost = 3.0 + (double)N * K / hbm;
+      if (few && p.cost < 3.0 + f * N * K / hbm) p.cost = 3.0 + f * N * K / hbm;
       if (p.cost < best.cost) best = p;
     }
   }
@@ -672,23 +691,27 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm) 
 //    least certain; 320 shapes up to 1024 rows: 11 % faster on average, 13 %
 //    slower at worst), else 5 %.  Up to 32 rows the strip, which reads A into
 //    registers, stays ahead.
-// ws: the call brings a workspace.  max_ws: the bytes of it that K-slices may
-// take (0: none).
+//  * Rows that do not start on 128-byte lines: 2, 7 and 16 % below, from the same
+//    fit as TileCost::ragged.
+// lines: as for tile_cost.  ws: the call brings a workspace.  max_ws: the bytes
+// of it that K-slices may take (0: none).
 constexpr int kNoTile = -1, kTile128 = -2, kTileNarrow = -3;
-int pick_tile(int M, int N, int K, int cus, bool ws, size_t max_ws, NarrowPlan* narrow) {
+int pick_tile(int M, int N, int K, int cus, bool lines, bool ws, size_t max_ws,
+              NarrowPlan* narrow) {
   if (M <= 32 || K <= 0 || N <= 0) return kNoTile;
-  const double named = named_cost(M, N, K, cus, ws);
+  const double named = named_cost(M, N, K, cus, ws, lines);
   int best = kNoTile;
   double cost = named;
   if (M > CfgSkinny::kMaxM) {
-    const double c128 = tile_cost(kCost128, M, N, K, cus);
-    if (c128 < 0.95 * named) {
+    const double ahead = (lines ? 0.95 : 0.98) * named;
+    const double c128 = tile_cost(kCost128, M, N, K, cus, lines);
+    if (c128 < ahead) {
       best = kTile128;
       cost = c128;
     }
     for (int t = 0; t < hk::kNumTiles; ++t) {
-      const double c = tile_cost(kCostMid[t], M, N, K, cus);
-      if (c < 0.95 * named && c < cost) {
+      const double c = tile_cost(kCostMid[t], M, N, K, cus, lines);
+      if (c < ahead && c < cost) {
         cost = c;
         best = t;
       }
@@ -700,8 +723,10 @@ int pick_tile(int M, int N, int K, int cus, bool ws, size_t max_ws, NarrowPlan* 
                       plan_t128(M, N, K, cus).slices > 1;
   // 5.3 TB/s measured; 4.6 against 128 x 128 tiles, whose own stream is as
   // fast there (over 100 MB of B_T).
-  *narrow = plan_narrow(M, N, K, cus, max_ws, t128 ? 4.6e6 : 5.3e6);
-  const double margin = M <= CfgSkinny::kMaxM ? 0.94 : ksplit ? 0.90 : 0.95;
+  *narrow = plan_narrow(M, N, K, cus, max_ws, t128 ? 4.6e6 : 5.3e6, lines);
+  const double margin = M <= CfgSkinny::kMaxM ? (lines ? 0.94 : 0.93)
+                        : ksplit              ? (lines ? 0.90 : 0.84)
+                                              : 0.95;
   return narrow->cost < margin * cost ? kTileNarrow : best;
 }
 
@@ -857,10 +882,11 @@ hipError_t run_gemm(const hipgemm_gemm_desc& d, bool ws_given,
     if (ws_given && ws_bytes < variant_ws(M, N, K, variant)) return hipErrorInvalidValue;
     const size_t most = narrow_max_ws(M, N, K, variant);
     const size_t max_ws = !ws_given ? 0 : ws_bytes < most ? ws_bytes : most;
-    int t = pick_tile(M, N, K, cu_count(), ws_given, max_ws, &np);
+    const bool lines = (lda | ldb) % 128 == 0 && aligned(d.A, 128) && aligned(d.B_T, 128);
+    int t = pick_tile(M, N, K, cu_count(), lines, ws_given, max_ws, &np);
     // fp32 and e4m3 outputs are not built for the 64-column K-slices.
     if (t == kTileNarrow && np.slices > 1 && key.out >= kOutF32)
-      t = pick_tile(M, N, K, cu_count(), ws_given, 0, &np);
+      t = pick_tile(M, N, K, cu_count(), lines, ws_given, 0, &np);
     // The tiles are not built for every epilogue: else what follows.
     hk::Key k = key;
     const void* fn = nullptr;
@@ -1141,14 +1167,14 @@ int hipgemm_split_columns(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int cus = cu_count();
   NarrowPlan np;
-  return pick_tile(M, N, K, cus, false, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
+  return pick_tile(M, N, K, cus, K % 128 == 0, false, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
 }
 
 int hipgemm_auto_tile(int M, int N, int K, int* bm, int* bn) {
   if (!bm || !bn) return 0;
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   NarrowPlan np;
-  const int t = pick_tile(M, N, K, cu_count(), true,
+  const int t = pick_tile(M, N, K, cu_count(), K % 128 == 0, true,
                           narrow_max_ws(M, N, K, hipgemm_select_variant(M, N, K)), &np);
   if (t == kNoTile) return 0;
   const hk::TileShape s = t == kTileNarrow ? hk::kNarrow[np.tile]
@@ -1267,7 +1293,7 @@ size_t hipgemm_workspace_size(int M, int N, int K, int variant) {
   if (v != named || K == 0) return variant_ws(M, N, K, v);
   // The schedule AUTO names covers AUTO's 64-column K-slices too.
   NarrowPlan np;
-  const int t = pick_tile(M, N, K, cu_count(), true, narrow_max_ws(M, N, K, v), &np);
+  const int t = pick_tile(M, N, K, cu_count(), K % 128 == 0, true, narrow_max_ws(M, N, K, v), &np);
   return auto_ws(M, N, K, v, t, np);
 }
 
