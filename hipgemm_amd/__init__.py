@@ -58,8 +58,9 @@ hipSuccess = 0
 hipErrorInvalidValue = 1
 
 
-class GemmDesc(ctypes.Structure):
-    """hipgemm_gemm_desc (include/hipgemm.h)."""
+class _Desc(ctypes.Structure):
+    """hipgemm_gemm_desc (include/hipgemm.h) from positional values: a call of
+    gemm() spent 7 us in GemmDesc's keyword loop, 1.5 here."""
     _fields_ = [("size", ctypes.c_size_t),
                 ("A", ctypes.c_void_p), ("B_T", ctypes.c_void_p),
                 ("C", ctypes.c_void_p),
@@ -78,17 +79,15 @@ class GemmDesc(ctypes.Structure):
                 ("mx_scale_b", ctypes.c_void_p),
                 ("scale_out", ctypes.c_void_p)]
 
+
+class GemmDesc(_Desc):
+    """hipgemm_gemm_desc (include/hipgemm.h)."""
+
     def __init__(self, **kw):
         super().__init__()
         self.size = ctypes.sizeof(GemmDesc)
         for k, v in kw.items():
             setattr(self, k, v or (None if k in _PTR_FIELDS else 0))
-
-
-class _Desc(ctypes.Structure):
-    """hipgemm_gemm_desc again, built from positional values: a call of gemm()
-    spent 7 us in GemmDesc's keyword loop, 1.5 here."""
-    _fields_ = GemmDesc._fields_
 
 
 _PTR_FIELDS = {"A", "B_T", "C", "scale_a", "scale_b", "scale_rows",
@@ -136,9 +135,9 @@ def lib() -> ctypes.CDLL:
                                                ci, vp, vp, ci, vp,
                                                ctypes.c_size_t, vp]
     L.hipgemm_fp8_gemm_bf16_rowcol.restype = ci
-    L.hipgemm_gemm.argtypes = [vp, vp]  # a hipgemm_gemm_desc by reference
+    L.hipgemm_gemm.argtypes = [ctypes.POINTER(_Desc), vp]
     L.hipgemm_gemm.restype = ci
-    L.hipgemm_gemm_noalloc.argtypes = [ctypes.POINTER(GemmDesc), vp]
+    L.hipgemm_gemm_noalloc.argtypes = [ctypes.POINTER(_Desc), vp]
     L.hipgemm_gemm_noalloc.restype = ci
     L.hipgemm_mx_scales_bytes.argtypes = [ci, ci]
     L.hipgemm_mx_scales_bytes.restype = ctypes.c_size_t
@@ -224,7 +223,7 @@ def gemm_raw_rowcol(a_ptr: int, b_ptr: int, c_ptr: int, M: int, N: int,
 
 def gemm_desc_raw(desc: "GemmDesc", stream: int = 0) -> int:
     """Call hipgemm_gemm; returns hipError_t."""
-    return int(lib().hipgemm_gemm(ctypes.addressof(desc), stream or None))
+    return int(lib().hipgemm_gemm(ctypes.byref(desc), stream or None))
 
 
 def gemm_desc_noalloc_raw(desc: "GemmDesc", stream: int = 0) -> int:
@@ -514,7 +513,7 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     d = _Desc(_DESC_BYTES, a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
               lda, ldb, ldc, a_format, b_format, codes[out_dtype],
               ACTIVATIONS[activation], *ptrs, variant, ws, nbytes, mx_a, mx_b, so)
-    _check(lib().hipgemm_gemm(ctypes.addressof(d), handle), "hipgemm_gemm")
+    _check(lib().hipgemm_gemm(d, handle), "hipgemm_gemm")
     return out
 
 

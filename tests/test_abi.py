@@ -461,3 +461,14 @@ def test_auto_picks_fit_their_shape_and_the_noalloc_scratch():
                 ws = hg.workspace_size(M, N, K, 0)
                 assert ws == hg.workspace_size(M, N, K, v), (M, N, K)
                 assert ws <= scratch, (M, N, K, v, ws)
+
+
+def test_descriptor_by_instance_or_reference():
+    """The bound functions take a descriptor itself or by reference, built from
+    keywords or positional values."""
+    L = hg.lib()
+    for d in (hg.GemmDesc(M=16, N=16, K=16), hg._Desc(hg._DESC_BYTES, 0, 0, 0, 16, 16, 16)):
+        assert d.size == ctypes.sizeof(hg.GemmDesc) and (d.M, d.N, d.K) == (16, 16, 16)
+        for arg in (d, ctypes.byref(d), ctypes.pointer(d)):
+            assert L.hipgemm_gemm(arg, None) == INVALID  # null C
+            assert L.hipgemm_gemm_noalloc(arg, None) == INVALID
