@@ -44,7 +44,17 @@ SHAPES = {
     (1537, 5392, 1040): (192, 128),  # several tiles per workgroup
     (2119, 4149, 16): (192, 128),    # odd N, two rounds, one K-step
     (2304, 2304, 1024): (192, 128),  # whole tiles and steps
+    (107, 17832, 32): (128, 64),     # one row of more tiles than workgroups:
+    (72, 20648, 128): (128, 64),     # on whole lines of B_T, each read once
+    (77, 17849, 16): (128, 64),      # odd N
+    (35, 34744, 1296): (64, 64),
+    (33, 35136, 1280): (64, 64),     # on whole lines of B_T
 }
+
+
+def tiles_of(shape):
+    (M, N, _), (bm, bn) = shape, SHAPES[shape]
+    return -(-M // bm) * -(-N // bn)
 
 
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
@@ -52,6 +62,12 @@ def test_auto_tile(shape):
     M, N, K = shape
     assert hg.auto_tile(M, N, K) == SHAPES[shape]
     assert hg.split_columns(M, N, K) == 0
+
+
+def test_shapes_cover_one_and_several_tiles_per_workgroup():
+    for tile in set(SHAPES.values()):
+        n = [tiles_of(s) for s in SHAPES if SHAPES[s] == tile]
+        assert min(n) <= 256 < max(n), tile
 
 
 def test_auto_tile_keeps_other_choices():
@@ -147,6 +163,55 @@ def test_tile_epilogue(gpu, oracle, shape, out):
                               scale_out=so or 1.0)
         runs(gpu, A, B, out, N + 8, want, fb=1, act=act, sa=[0.5], sr=sr, sc=sc,
              bias=bias, so=None if so is None else [so])
+
+
+# Largest step between neighbouring values, relative, and the smallest value that
+# it holds down to.
+STEP = {po.OUT_BF16: (2.0 ** -7, 2.0 ** -126), po.OUT_F16: (2.0 ** -10, 2.0 ** -14),
+        po.OUT_F32: (1e-5, 0.0), po.OUT_FP8: (2.0 ** -3, 2.0 ** -6)}
+
+
+def values(torch, bits, out):
+    dt = {po.OUT_BF16: torch.bfloat16, po.OUT_F16: torch.float16,
+          po.OUT_F32: torch.float32, po.OUT_FP8: torch.float8_e4m3fn}[out]
+    return torch.from_numpy(bits.view({4: np.int32, 2: np.int16, 1: np.uint8}[ES[out]])
+                            ).view(dt).double().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("act", [po.ACT_SILU, po.ACT_GELU_TANH], ids=["silu", "gelu"])
+@pytest.mark.parametrize("shape", [
+    (33, 200, 4096), (200, 6144, 640), (72, 20648, 128), (4221, 1832, 16),
+    (2055, 3640, 336), (2304, 3840, 512), (1237, 3280, 592)],
+    ids=lambda s: "x".join(map(str, s)))
+def test_tile_transcendental(gpu, oracle, shape, act):
+    """silu and gelu on every tile and output type.  The values before the
+    activation are exact; it is evaluated with an exponential of relative error
+    2^-24 |log2| (|log2| < 100 here) and a reciprocal: fp32 within 1e-5, the other
+    types at most one step apart, and equal but for values that close to a
+    midpoint (1e-5 of 2^-8 at the most: under 1 %).  2^-46 for the oracle's 1 +
+    tanh, which cancels in double precision (|v| 2^-52, |v| < 2^6)."""
+    M, N, K = shape
+    rng = np.random.default_rng(9)
+    A, B = TERN[0][rng.integers(0, 3, (M, K))], TERN[0][rng.integers(0, 3, (N, K))]
+    sa = 2.0 ** -round(np.log2(K ** 0.5 * 0.5))  # standard deviation about 1.3
+    bias = rng.integers(-8, 9, N).astype(np.float32) / 8
+    need = hg.workspace_size(M, N, K, 0)
+    for out in ES:
+        say(f"case tile {SHAPES[shape]} M={M} N={N} K={K} out={out} act={act}")
+        so = 4.0 if out == po.OUT_FP8 else None
+        want = oracle.gemm_ex(A, B, out=out, act=act, scale_a=sa, bias=bias,
+                              scale_out=so or 1.0)
+        r = values(gpu, want, out)
+        for ws in (0, need) if need else (0,):
+            w = gpu.zeros(ws, dtype=gpu.uint8, device="cuda") if ws else None
+            C, guard = run(gpu, A, B, out, N + 8, act=act, sa=[sa], bias=bias,
+                           so=None if so is None else [so], ws=w)
+            assert guard, "write outside M x N"
+            step, least = STEP[out]
+            c = values(gpu, C, out)
+            assert np.all(np.abs(c - r) <= step * np.maximum(np.abs(r), least) + 2.0 ** -46)
+            assert out == po.OUT_F32 or np.mean(C == want) > 0.99
 
 
 @pytest.mark.gpu
