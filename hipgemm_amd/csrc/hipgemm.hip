@@ -549,10 +549,10 @@ int split_columns(int M, int N, int cus) {
 // every tile timed on each: 5-9 % standard error per tile.
 // ragged: how much longer the steps take where rows do not start on 128-byte
 // lines, so that a step's part of a row lies in two.  These factors and the ones
-// below come from 1100 such shapes from 33 rows up, operands from memory: without
-// them 97 of 2100 choices were more than 3 % behind the named schedule (64 x 64
-// tiles, 55 x 16472 x 13744 106 against 86 us), with them 42, and all together
-// 1.0 % behind the fastest instead of 1.25.
+// below come from 1900 such shapes from 33 rows up with operands from memory.  On
+// 2450 other calls (all outputs, with and without a workspace) 62 are more than 3 %
+// behind the named schedules, 182 without the factors (55 x 16472 x 13744 106
+// against 86 us, 64 x 1024 x 4112 11.1 / 8.8).
 struct TileCost {
   int bm, bn;
   double launch, round, step, busy, ragged;
@@ -571,6 +571,9 @@ double tile_cost(const TileCost& c, int M, int N, int K, int cus, bool lines) {
              (c.step * rounds + c.busy * tiles / cus);
 }
 
+// Up to 128 rows the steps are streams over B_T, all as much longer.
+constexpr double kRaggedFew = 1.6;
+
 // Cost of what hipgemm_select_variant and hipgemm_split_columns name for 33
 // rows and more (the same model; the strip's per step the bytes of its columns
 // and of A's row blocks; 5-7 % standard error on 146 and 135 shapes up to 128
@@ -582,7 +585,7 @@ double named_cost(int M, int N, int K, int cus, bool ws, bool lines) {
     const double w = p.knb / 2.0, area = p.kmb * p.knb / 8.0;
     const int rounds = ceil_div(p.tiles_n * p.slices, cus);
     return 3.54 +
-           (lines ? 1.0 : 1.27) * p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) +
+           (lines ? 1.0 : kRaggedFew) * p.slice_steps * rounds * (0.114 * w + 0.111 * p.kmb / 4) +
            1.10 * area +
            (p.slices > 1 ? 2.02 + 0.189 * p.slices * area : 0.0);
   }
@@ -596,7 +599,8 @@ double named_cost(int M, int N, int K, int cus, bool ws, bool lines) {
     if (!ws) return 1e9;
     const SkinnyPlan p = plan_skinny(M, N, K);
     const int units = p.tiles_n * p.slices;
-    return 7.9 + 0.57 * ceil_div(units, cus) * p.slice_steps * p.bn / 128 + 5.3 * units / cus;
+    return (lines ? 1.0 : 1.14) * (7.9 + 0.57 * ceil_div(units, cus) * p.slice_steps * p.bn / 128 +
+                                   5.3 * units / cus);
   }
   const int n1 = split_columns(M, N, cus);
   if (n1 > 0)
@@ -604,7 +608,7 @@ double named_cost(int M, int N, int K, int cus, bool ws, bool lines) {
            0.91 * tile_cost(kCost128, M, N - n1, K, cus, lines);
   if (variant != HIPGEMM_VARIANT_TILE128)
     return tile_cost(kCost256, M, N, K, cus, lines);
-  const double f = lines ? 1.0 : 1.14;
+  const double f = lines ? 1.0 : M <= CfgSkinny::kMaxM ? kRaggedFew : 1.14;
   const T128Plan ks = plan_t128(M, N, K, cus);
   const double units = (double)ceil_div(M, 128) * ceil_div(N, 128) * ks.slices / cus;
   if (M <= CfgSkinny::kMaxM) {
@@ -639,19 +643,23 @@ constexpr NarrowCost kNarrowFew[hk::kNumNarrow] = {
 constexpr NarrowCost kNarrowMany[hk::kNumNarrow] = {
     {3.04, 0.89, 0.236, 0.119, 0.68, 2.77, 0.787},
     {2.92, 0.82, 0.156, 0.075, 0.96, 1.04, 0.607}};
-// As TileCost::ragged, over whole K and in slices.
+// As TileCost::ragged above 128 rows, over whole K and in slices.
 constexpr double kNarrowRagged = 1.20, kSlicesRagged = 1.10;
 // The cheapest plan: K-slices of at least 8 steps, at most one workgroup per
 // CU, within max_ws bytes of workspace.  hbm: bytes per us that a stream of B_T
-// under one row of tiles reaches.
+// under one row of tiles reaches.  t128: the named schedule is the 128 x 128 one.
 NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm,
-                       bool lines) {
+                       bool lines, bool t128) {
   NarrowPlan best;
   const int steps = ceil_div(K, 128);
   for (int t = 0; t < hk::kNumNarrow; ++t) {
     const bool few = M <= CfgSkinny::kMaxM;
     const NarrowCost& c = few ? kNarrowFew[t] : kNarrowMany[t];
     const int tiles = ceil_div(M, hk::kNarrow[t].bm) * ceil_div(N, hk::kNarrow[t].bn);
+    // One row of tiles in more than one round: behind the 128 x 128 tiles' one round
+    // where those are named (64 x 64 tiles 7 %, 128 x 64 15 % on average over 211
+    // shapes; 49 x 17184 x 11008 54.8 against 48.0 us).
+    if (t128 && M <= hk::kNarrow[t].bm && tiles > cus) continue;
     for (int s = 1; s <= 8; ++s) {
       if (s > 1 && (tiles * s > cus || 8 * s > steps)) break;
       NarrowPlan p;
@@ -660,7 +668,10 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm,
       p.slices = ceil_div(steps, p.slice_steps);
       const int units = tiles * p.slices, rounds = ceil_div(units, cus);
       const double share = (double)units / cus;
-      const double f = lines ? 1.0 : p.slices > 1 ? kSlicesRagged : kNarrowRagged;
+      const double f = lines          ? 1.0
+                       : few          ? kRaggedFew
+                       : p.slices > 1 ? kSlicesRagged
+                                      : kNarrowRagged;
       p.cost = c.launch + c.round * rounds +
                f * p.slice_steps * (c.step * rounds + c.busy * share);
       if (p.slices > 1) {
@@ -691,8 +702,8 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm,
 //    least certain; 320 shapes up to 1024 rows: 11 % faster on average, 13 %
 //    slower at worst), else 5 %.  Up to 32 rows the strip, which reads A into
 //    registers, stays ahead.
-//  * Rows that do not start on 128-byte lines: 2, 7 and 16 % below, from the same
-//    fit as TileCost::ragged.
+//  * Rows that do not start on 128-byte lines: 2, 7 (9 up to 64 rows) and 16 %
+//    below, from the same fit as TileCost::ragged.
 // lines: as for tile_cost.  ws: the call brings a workspace.  max_ws: the bytes
 // of it that K-slices may take (0: none).
 constexpr int kNoTile = -1, kTile128 = -2, kTileNarrow = -3;
@@ -723,8 +734,8 @@ int pick_tile(int M, int N, int K, int cus, bool lines, bool ws, size_t max_ws,
                       plan_t128(M, N, K, cus).slices > 1;
   // 5.3 TB/s measured; 4.6 against 128 x 128 tiles, whose own stream is as
   // fast there (over 100 MB of B_T).
-  *narrow = plan_narrow(M, N, K, cus, max_ws, t128 ? 4.6e6 : 5.3e6, lines);
-  const double margin = M <= CfgSkinny::kMaxM ? (lines ? 0.94 : 0.93)
+  *narrow = plan_narrow(M, N, K, cus, max_ws, t128 ? 4.6e6 : 5.3e6, lines, t128);
+  const double margin = M <= CfgSkinny::kMaxM ? (lines ? 0.94 : M <= 64 ? 0.91 : 0.93)
                         : ksplit              ? (lines ? 0.90 : 0.84)
                                               : 0.95;
   return narrow->cost < margin * cost ? kTileNarrow : best;

@@ -1,5 +1,5 @@
-"""Schedule sweep: time every applicable schedule on given shapes and report
-AUTO's pick against the fastest.
+"""Schedule sweep: time AUTO and every applicable schedule on given shapes and
+report AUTO against the fastest.
 
     python -m hipgemm_amd.sweep 64x4096x4096,128x8192x8192 [--variants 3,5,6]
     python -m hipgemm_amd.sweep --grid 16,32:4096,8192:2048,8192 \
@@ -8,14 +8,15 @@ AUTO's pick against the fastest.
 For each M x N x K: e4m3 operands drawn from normal(0, 1) (rotating sets
 of at least 512 MiB, so that the L2 and the MALL do not hold them between
 launches), per-tensor scales, bf16 C, one caller workspace
-(hipgemm_fp8_gemm_bf16_ws).  The schedules are timed in alternating blocks
-of launches (four rounds, the order reversed every other round) with HIP
-events on one stream; a schedule that rejects the shape is left out.  One
-line per shape: microseconds per launch for each schedule, AUTO's pick
-(hipgemm_select_variant; for AUTO's column split the 4-wave schedule is
-reported), the fastest, and AUTO's time over the fastest (with
---show-above R, only the shapes whose ratio exceeds R).  The summary gives
-the mean and worst ratio and how many shapes fall in each ratio bucket.
+(hipgemm_fp8_gemm_bf16_ws).  AUTO (variant 0, whatever it runs) and the
+schedules are timed in alternating blocks of launches (four rounds, the order
+reversed every other round) with HIP events on one stream; a schedule that
+rejects the shape is left out.  One line per shape: microseconds per launch for
+each, the schedule that AUTO names (hipgemm_select_variant) and its own tile
+where it runs another (hipgemm_auto_tile), the fastest, and AUTO's time over the
+fastest (with --show-above R, only the shapes whose ratio exceeds R).  The
+summary gives the mean and worst ratio and how many shapes fall in each ratio
+bucket.
 --grid M,..:N,..:K,.. adds every combination of the listed sizes.
 
 Measurement only: it checks no results (the tests do).
@@ -25,7 +26,7 @@ from __future__ import annotations
 import argparse
 import sys
 
-from . import VARIANTS, lib, variant_name, workspace_size
+from . import VARIANTS, auto_tile, lib, variant_name, workspace_size
 
 
 def parse_shapes(text: str):
@@ -60,6 +61,8 @@ def sweep(shapes, variants, rounds: int = 4, launches: int = 100, out=sys.stdout
     torch.cuda.set_device(dev)
     stream = torch.cuda.current_stream()
     L = lib()
+    AUTO = VARIANTS["auto"]
+    variants = [AUTO] + [v for v in variants if v != AUTO]
     ratios = []
     for (M, N, K) in shapes:
         nsets = max(1, -(-(512 << 20) // (M * K + N * K)))
@@ -105,18 +108,16 @@ def sweep(shapes, variants, rounds: int = 4, launches: int = 100, out=sys.stdout
                 e1.record(stream)
                 torch.cuda.synchronize()
                 us[v] += e0.elapsed_time(e1) * 1000.0 / launches / rounds
-        auto = int(L.hipgemm_select_variant(M, N, K))
         best = min(us, key=us.get)
-        line = "  ".join(f"{variant_name(v)} {us[v]:.2f}" for v in ok)
-        ratio = None
-        if auto in us:
-            ratio = us[auto] / us[best]
-            ratios.append(ratio)
-            tail = f"auto={variant_name(auto)} best={variant_name(best)} ratio {ratio:.3f}"
-        else:
-            tail = f"auto={variant_name(auto)} (not timed) best={variant_name(best)}"
-        if ratio is None or ratio > show_above:
-            print(f"{M}x{N}x{K}: {line}  | {tail}", file=out, flush=True)
+        ratio = us[AUTO] / us[best]
+        ratios.append(ratio)
+        own = auto_tile(M, N, K)
+        named = variant_name(int(L.hipgemm_select_variant(M, N, K)))
+        if ratio > show_above:
+            print(f"{M}x{N}x{K}: " +
+                  "  ".join(f"{variant_name(v)} {us[v]:.2f}" for v in ok) +
+                  f"  | names {named}" + (f", runs {own[0]}x{own[1]} tiles" if own else "") +
+                  f"  best={variant_name(best)} ratio {ratio:.3f}", file=out, flush=True)
         del As, Bs, C, ws
     if ratios:
         print(f"summary: {len(ratios)} shapes, AUTO / fastest mean "

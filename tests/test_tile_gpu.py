@@ -47,8 +47,6 @@ SHAPES = {
     (107, 17832, 32): (128, 64),     # one row of more tiles than workgroups:
     (72, 20648, 128): (128, 64),     # on whole lines of B_T, each read once
     (77, 17849, 16): (128, 64),      # odd N
-    (35, 34744, 1296): (64, 64),
-    (33, 35136, 1280): (64, 64),     # on whole lines of B_T
 }
 
 
@@ -65,9 +63,21 @@ def test_auto_tile(shape):
 
 
 def test_shapes_cover_one_and_several_tiles_per_workgroup():
+    """(AUTO runs 64 x 64 tiles in one round only.)"""
     for tile in set(SHAPES.values()):
         n = [tiles_of(s) for s in SHAPES if SHAPES[s] == tile]
-        assert min(n) <= 256 < max(n), tile
+        assert min(n) <= 256 and (max(n) > 256) == (tile != (64, 64)), tile
+
+
+def test_one_row_of_64_column_tiles_in_one_round():
+    """Where 128 x 128 tiles are named, more 64-column tiles than CUs in one row
+    are not taken; where strips are, they may be."""
+    for M in (33, 48, 64):
+        for N in (16448, 17408, 24576, 32768):
+            for K in (1024, 4096, 8208, 11008):
+                assert hg.select_variant(M, N, K) == hg.VARIANTS["tile128"]
+                assert hg.auto_tile(M, N, K) is None, (M, N, K)
+    assert hg.select_variant(107, 17832, 32) == hg.VARIANTS["strip"]
 
 
 def test_auto_tile_keeps_other_choices():
