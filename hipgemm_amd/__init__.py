@@ -480,7 +480,8 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     if b_t.dtype == torch.float4_e2m1fn_x2:
         b_t = b_t.view(torch.uint8)
     out_dtype = out_dtype or (out.dtype if out is not None else torch.bfloat16)
-    if out_dtype not in codes:
+    out_code = codes.get(out_dtype)
+    if out_code is None:
         raise HipGemmError("out_dtype must be bfloat16, float16, float32 or "
                            "float8_e4m3fn", hipErrorInvalidValue)
     if activation not in ACTIVATIONS:
@@ -508,10 +509,9 @@ def gemm(a, b_t, *, a_format: int = FMT_E4M3, b_format: int = FMT_E4M3,
     so = _scale_ptr(scale_out, "scale_out")
     ws, nbytes = _stream_workspace(
         a, stream, handle, _ws_bytes(a.get_device(), M, N, K, variant, a_format,
-                                     b_format, bool(mx_a or mx_b),
-                                     codes[out_dtype]))
+                                     b_format, bool(mx_a or mx_b), out_code))
     d = _Desc(_DESC_BYTES, a.data_ptr(), b_t.data_ptr(), out.data_ptr(), M, N, K,
-              lda, ldb, ldc, a_format, b_format, codes[out_dtype],
+              lda, ldb, ldc, a_format, b_format, out_code,
               ACTIVATIONS[activation], *ptrs, variant, ws, nbytes, mx_a, mx_b, so)
     _check(lib().hipgemm_gemm(d, handle), "hipgemm_gemm")
     return out
