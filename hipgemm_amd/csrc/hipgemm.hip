@@ -550,8 +550,8 @@ int split_columns(int M, int N, int cus) {
 // ragged: how much longer the steps take where rows do not start on 128-byte
 // lines, so that a step's part of a row lies in two.  These factors and the ones
 // below come from 1900 such shapes from 33 rows up with operands from memory.  On
-// 2450 other calls (all outputs, with and without a workspace) 62 are more than 3 %
-// behind the named schedules, 182 without the factors (55 x 16472 x 13744 106
+// 2200 other calls (all outputs, with and without a workspace) 47 are more than 3 %
+// behind the named schedules, 170 without the factors (55 x 16472 x 13744 106
 // against 86 us, 64 x 1024 x 4112 11.1 / 8.8).
 struct TileCost {
   int bm, bn;
@@ -628,10 +628,12 @@ double named_cost(int M, int N, int K, int cus, bool ws, bool lines) {
 // such streams whatever is in flight (a DMA-only loop), so that A's rows, read
 // again by every column of tiles, count as much as B_T's; and with K-slices
 // half the fp32 partials of 128 x 128 tiles go out and come back, the last
-// arrivals that sum them spread over twice the CUs.  Us, before -> after: 128 x
-// 8192 x 8192 (2 slices) 22.5 -> 20.9, 128 x 14336 x 4096 23.4 -> 17.7, 128 x
-// 8192 x 2048 13.6 -> 8.2, 64 x 8192 x 8192 (64 x 64, 2 slices) 21.0 -> 16.3,
-// 64 x 14336 x 4096 17.9 -> 13.8, 256 x 4096 x 4096 (64 x 64) 19.0 -> 11.7.
+// arrivals that sum them spread over twice the CUs.  Us per call, operands from
+// memory, before -> after: 128 x 8192 x 8192 (2 slices) 22.8 -> 21.2 (21.2 -> 17.4
+// on one set of operands, which the last-level cache holds), 128 x 14336 x 4096
+// 23.7 -> 17.8, 128 x 8192 x 2048 13.8 -> 8.5, 64 x 8192 x 8192 (64 x 64, 2 slices)
+// 20.8 -> 16.6, 64 x 14336 x 4096 17.8 -> 14.0, 256 x 4096 x 4096 (64 x 64) 18.4 ->
+// 12.5.
 // Model as above plus the slices' terms, fitted apart up to 128 rows and above
 // (7 % standard error over 440 and 320 shapes, every plan timed).
 struct NarrowCost {
@@ -692,10 +694,11 @@ NarrowPlan plan_narrow(int M, int N, int K, int cus, size_t max_ws, double hbm,
 // hk::kTiles, kTile128 (128 x 128, no K-split), kTileNarrow (`narrow`), or
 // kNoTile.
 //  * Above 128 rows the tiles between 128 x 128 and 256 x 256, 5 % below the
-//    named cost: over 298 shapes 6 % faster on average (2048 x 4096 x 4096 37.3
-//    -> 26.5 us, 3072^3 28.7 -> 23.3, 1536 x 4096 x 4096 28.9 -> 20.0, 1024 x
-//    8192 x 4096 38 -> 30.5, 1024 x 1024 x 4096 19.2 -> 14.3), one slower by
-//    more than 3 % (5.7 %); without the margin eight.
+//    named cost: over 298 shapes 6 % faster on average, one slower by more than
+//    3 % (5.7 %); without the margin eight.  Operands from memory, us: 2048 x 4096 x
+//    4096 40.2 -> 31.5, 3072^3 33.8 -> 27.4, 1536 x 4096 x 4096 35.2 -> 24.8, 1024 x
+//    8192 x 4096 40.7 -> 31.2, 1024 x 1024 x 4096 19.4 -> 11.5.  Most of the calls
+//    that lose have over 20000 columns (382 x 27824 x 6144 67.6 -> 77.9).
 //  * 64-column tiles up to 1024 rows: 6 % below from 33 to 128 rows (277
 //    shapes: 17 % faster on average, three slower by more than 3 %, 10 % at
 //    worst), 10 % below a K-split of 128 x 128 tiles above (its cost is the
@@ -1178,7 +1181,9 @@ int hipgemm_split_columns(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int cus = cu_count();
   NarrowPlan np;
-  return pick_tile(M, N, K, cus, K % 128 == 0, false, 0, &np) == kNoTile ? split_columns(M, N, cus) : 0;
+  return pick_tile(M, N, K, cus, K % 128 == 0, false, 0, &np) == kNoTile
+             ? split_columns(M, N, cus)
+             : 0;
 }
 
 int hipgemm_auto_tile(int M, int N, int K, int* bm, int* bn) {

@@ -52,7 +52,12 @@ extern "C" {
  * workspace serves calls of every shape and schedule in turn. */
 #define HIPGEMM_WS_COUNTER_BYTES 16384
 
-/* Schedules.  AUTO picks by shape (hipgemm_select_variant). */
+/* Schedules.  AUTO names one by shape (hipgemm_select_variant: "AUTO's choice"
+ * below) and runs it, except that 8-bit operands without MX scales from 33 rows
+ * up run on another tile of the 128 x 128 schedule's loop where one is estimated
+ * faster (hipgemm_auto_tile: most calls from 33 to 128 rows and many above; so
+ * SKINNY seldom runs but where those tiles are not built, or for fp32 and e4m3
+ * outputs with few columns and long rows). */
 enum {
   HIPGEMM_VARIANT_AUTO = 0,
   /* 256 threads (4 waves, one per SIMD), 256 x 256 tile, 2 LDS stages,
@@ -377,15 +382,18 @@ hipError_t hipgemm_fp8_gemm_4wave_256x256x128(const void *A, const void *B_T,
                                               void *C, int M, int N, int K,
                                               hipStream_t stream);
 
-/* Variant AUTO resolves to for this shape (no GPU needed). No reference
- * counterpart (the reference has one schedule). */
+/* The schedule that AUTO names for this shape (no GPU needed); where
+ * hipgemm_auto_tile returns 1, 8-bit operands run on that tile instead.  No
+ * reference counterpart (the reference has one schedule). */
 int hipgemm_select_variant(int M, int N, int K);
 
 /* AUTO's column split: when the last round of 256 x 256 tiles would leave
  * most CUs idle, AUTO runs columns [0, n1) of C on the 4-wave 16x16x128
  * schedule (whole rounds) and [n1, N) on the 128 x 128 schedule, two
  * launches on the caller's stream.  Returns n1 (a multiple of 256), or 0
- * when AUTO runs one schedule.  Uses the current device's CU count (256
+ * when AUTO runs one schedule, or the tile of hipgemm_auto_tile (calls that that
+ * tile is not built for, extended epilogues without aligned stores, may still
+ * split).  Uses the current device's CU count (256
  * without a device).  No reference counterpart (the reference's grid is
  * M*N/65536 tiles of 256 x 256, fp8_4wave.hpp:357-377). */
 int hipgemm_split_columns(int M, int N, int K);
@@ -398,8 +406,9 @@ int hipgemm_split_columns(int M, int N, int K);
  * 1024 rows, on 128 x 64 or 64 x 64 tiles -- those in K-slices where that is
  * faster and the call brings a workspace that holds them (what
  * hipgemm_workspace_size names for AUTO does) or runs hipgemm_gemm_noalloc, the
- * last slice to arrive at a part of a tile summing it.  No reference counterpart (the reference has 256 x 256
- * tiles only). */
+ * last slice to arrive at a part of a tile summing it.  For packed operands (lda =
+ * ldb = K): the choice also depends on whether rows start on 128-byte lines.  No
+ * reference counterpart (the reference has 256 x 256 tiles only). */
 int hipgemm_auto_tile(int M, int N, int K, int *bm, int *bn);
 
 /* Human-readable variant name, or NULL.  No reference counterpart. */

@@ -18,10 +18,11 @@
 // 32 cycles per wave; on 128 x 128 these take 0.33, 0.35 and 0.23 us, a step
 // 0.39 us.  With one select and one address computation per DMA and per
 // read in the loop, and the wave's scalar work after the barrier, a step was
-// 0.47 us (2048 x 2048 x 8192 34.2 -> 29.9 us, 1536 x 4096 x 4096 33.0 ->
-// 28.9, 1024^3 7.45 -> 7.10, MXFP4 2048 x 2048 x 8192 25.0 -> 22.9, with row
-// and column scales, bias and silu 2048 x 2048 x 4096 23.0 -> 19.2): the
-// steady loop now has four address additions per step and nothing else.
+// 0.47 us (one set of operands: 2048 x 2048 x 8192 34.2 -> 29.9 us, 1536 x 4096 x
+// 4096 33.0 -> 28.9, 1024^3 7.45 -> 7.10, MXFP4 2048 x 2048 x 8192 25.0 -> 22.9,
+// with row and column scales, bias and silu 2048 x 2048 x 4096 23.0 -> 19.2;
+// operands from memory: the first two 39.0 -> 36.8 and 35.0 -> 31.8): the steady
+// loop now has four address additions per step and nothing else.
 //
 // Pipeline: S LDS stages of BM + BN rows x 128 bytes, DMA'd (buffer_load_dwordx4
 // ... lds) S steps ahead of the reads, and two register sets: the fragments
@@ -47,29 +48,29 @@
 // of a step falls at the same offset of each operand row, and with row strides
 // that are a multiple of 4096 bytes all those rows meet at one offset within
 // 4 KiB -- which measured as an HBM-bound stall; one start per XCD keeps the
-// workgroups of an XCD (which share operand panels in their L2) in step.  Same process, 128 x 128 tiles,
-// against starting at step 0: 40 x 28672 x 4096 +19 %, 16 x 28672 x 4096
-// +24 %, 64 x 16384 x 8192 +29 %, 4096 x 1536 x 4096 +5 %, 512 x 4096 x 8192
-// and 2048 x 2048 x 8192 within 1 %.  The fp32 sums run in that rotated order
-// (deterministic per launch shape).
+// workgroups of an XCD (which share operand panels in their L2) in step.  Same
+// process, 128 x 128 tiles, against starting at step 0: 40 x 28672 x 4096 +19 %,
+// 16 x 28672 x 4096 +24 %, 64 x 16384 x 8192 +29 %, 4096 x 1536 x 4096 +5 %, 512 x
+// 4096 x 8192 and 2048 x 2048 x 8192 within 1 %; K-slices that are not all whole
+// steps 407 x 3072 x 11648 +9 %, 1006 x 3072 x 5824 +7 %.  The fp32 sums run in
+// that rotated order (deterministic per launch shape).
 //
 // LDS layout: 128-byte rows with the slot_xor swizzle, lane group g reading
 // slots 2g and 2g + 1 before the XOR (layout.hpp: conflict-free; A and B_T
 // share the K order).  kMx needs the instruction's own K order: chunks g and
 // g + 4 under strip_xor, conflict-free too.
 //
-// kSplit (128 x 128 tiles): work units are (tile, K-slice) pairs (g.split);
-// each writes its fp32 partial tile (written through to the coherent level,
-// sc1: the slices of a tile run on several XCDs, whose L2s are not coherent
+// kSplit (128 x 128 and 64-column tiles): work units are (tile, K-slice) pairs
+// (g.split); each writes its fp32 partial tile (written through to the coherent
+// level, sc1: the slices of a tile run on several XCDs, whose L2s are not coherent
 // with each other).  With g.split.arrivals, each wave then waits for its own
-// partial stores, counts its quadrant's arrival (a relaxed agent-scope
-// atomic), and the wave that arrives last at a quadrant sums the quadrant's
-// partials in slice order (its own from its accumulators, the others read
-// back with sc1) and runs the epilogue on the sum: no waiting on other
-// workgroups and no barrier, so waves of one workgroup may take different
-// paths here.  Without it, gemm_t128_reduce_body sums them in a kernel of its
-// own; both add +0 + slice 0 + slice 1 + ... in fp32, so their outputs are the
-// same.
+// partial stores, counts its quadrant's arrival (a relaxed agent-scope atomic),
+// and the wave that arrives last at a quadrant sums the quadrant's partials in
+// slice order (its own from its accumulators, the others read back with sc1) and
+// runs the epilogue on the sum: no waiting on other workgroups and no barrier, so
+// waves of one workgroup may take different paths here.  Without it,
+// gemm_t128_reduce_body sums them in a kernel of its own; both add +0 + slice 0 +
+// slice 1 + ... in fp32, so their outputs are the same.
 //
 // kNt: B_T's DMA carry the non-temporal hint, for one row of tiles, where each
 // B_T line is read by one workgroup (64 x 14336 x 4096 on 64 x 64 tiles 14.9 ->
